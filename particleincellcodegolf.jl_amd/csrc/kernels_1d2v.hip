@@ -23,15 +23,28 @@ namespace pic {
 template <int R>
 __device__ __forceinline__ void deposit_gauss_q(u64* __restrict__ acc, int32_t N, double c, double Nd,
                                                 int32_t nmask, double q, double w, int qb) {
-    const int64_t i0 = (int64_t)rint(c * Nd);
-    double prev = edge_half_erf(i0 - R, c, Nd);
+    const double cN = c * Nd, i0d = rint(cN);
+    if (!edges_fit(cN) || !limbs_fit(q * w, qb)) {
+        const int64_t i0 = (int64_t)i0d;
+        double prev = edge_half_erf(i0 - R, c, Nd);
 #pragma unroll 1
+        for (int j = -R; j <= R; ++j) {
+            const double next = edge_half_erf(i0 + j + 1, c, Nd);
+            const double wt = next - prev;
+            prev = next;
+            const double a = (q * wt) * w;
+            if (a != 0.0) lds_add_fxp(acc, N, cell0(i0 + j, nmask), fxp_from(fabs(a), qb));
+        }
+        return;
+    }
+    double f[2 * R + 2];
+    gauss_edges<R>(c, i0d, Nd, 1.0 / Nd, f);
+    const int32_t i0 = (int32_t)(int64_t)i0d;
+#pragma unroll
     for (int j = -R; j <= R; ++j) {
-        const double next = edge_half_erf(i0 + j + 1, c, Nd);
-        const double wt = next - prev;
-        prev = next;
-        const double a = (q * wt) * w;
-        if (a != 0.0) lds_add_fxp(acc, N, cell0(i0 + j, nmask), fxp_from(fabs(a), qb));
+        if (j == -7 || j == 7) continue;  // both edges beyond 6: the weight is exactly 0
+        const double wt = f[j + R + 1] - f[j + R];
+        lds_add_contribution(acc, N, (i0 + j - 1) & nmask, (q * wt) * w, qb);
     }
 }
 

@@ -3,6 +3,7 @@
 // and device-scope charge accumulators, and the loop-state predicates of the
 // step graph.  Compiled with -ffp-contract=off by every includer.
 #pragma once
+#include "gauss_edges.h"
 #include "pic_device.h"
 #include "pic_internal.h"
 
@@ -13,39 +14,81 @@ namespace pic {
 // Stencil helpers (R = 6 or 7)
 // ---------------------------------------------------------------------------
 
+// Whether gauss_edges may evaluate a centre: finite and near enough for exact
+// cell arithmetic in doubles
+__device__ __forceinline__ bool edges_fit(double cN) { return fabs(cN) < 0x1p51; }
+
 // S = sum(k -> E[k[1]]*k[2], d(c)) as a left fold over the 2R+1 cells
 // (src/GaussianFixedPointQuiet.jl:10); E is staged in LDS.
 template <int R>
 __device__ __forceinline__ double gather_gauss(const double* __restrict__ Eld, double c,
                                                double Nd, int32_t nmask) {
-    const int64_t i0 = (int64_t)rint(c * Nd);
-    double prev = edge_half_erf(i0 - R, c, Nd);
-    double S = 0.0;
+    const double cN = c * Nd, i0d = rint(cN);
+    if (!edges_fit(cN)) {
+        const int64_t i0 = (int64_t)i0d;
+        double prev = edge_half_erf(i0 - R, c, Nd);
+        double S = 0.0;
 #pragma unroll 1
+        for (int j = -R; j <= R; ++j) {
+            double next = edge_half_erf(i0 + j + 1, c, Nd);
+            double wt = next - prev;
+            prev = next;
+            double term = Eld[cell0(i0 + j, nmask)] * wt;
+            S = (j == -R) ? term : S + term;
+        }
+        return S;
+    }
+    double f[2 * R + 2];
+    gauss_edges<R>(c, i0d, Nd, 1.0 / Nd, f);
+    const int32_t i0 = (int32_t)(int64_t)i0d;
+    double S = 0.0;
+#pragma unroll
     for (int j = -R; j <= R; ++j) {
-        double next = edge_half_erf(i0 + j + 1, c, Nd);
-        double wt = next - prev;
-        prev = next;
-        double term = Eld[cell0(i0 + j, nmask)] * wt;
+        const double wt = f[j + R + 1] - f[j + R];
+        const double term = Eld[(i0 + j - 1) & nmask] * wt;
         S = (j == -R) ? term : S + term;
     }
     return S;
 }
+
+// |a| on the 2^-q grid, added into the LDS limbs of a cell: the limbs of
+// fxp_from, split exactly in doubles.  For |a| 2^q < 2^126 (limbs_fit).
+__device__ __forceinline__ void lds_add_contribution(u64* __restrict__ acc, int32_t N, int32_t cell, double a, int q) {
+    const Limbs43 v = split43(ldexp(fabs(a), q));
+    if (v.l0 != 0.0) atomicAdd(&acc[cell], small_u64(v.l0));
+    if (v.l1 != 0.0) atomicAdd(&acc[N + cell], small_u64(v.l1));
+    if (v.l2 != 0.0) atomicAdd(&acc[2 * N + cell], small_u64(v.l2));
+}
+// contributions of at most |w| each (uniform over a launch)
+__device__ __forceinline__ bool limbs_fit(double w, int q) { return ldexp(fabs(w), q) < 0x1p125; }
 
 // r[k[1]] += k[2]*w for the 2R+1 cells of d(c) (src/GaussianFixedPointQuiet.jl:7),
 // each product rounded to the 2^-q integer grid and added into LDS limbs.
 template <int R>
 __device__ __forceinline__ void deposit_gauss(u64* __restrict__ acc, int32_t N, double c,
                                               double Nd, int32_t nmask, double w, int q) {
-    const int64_t i0 = (int64_t)rint(c * Nd);
-    double prev = edge_half_erf(i0 - R, c, Nd);
+    const double cN = c * Nd, i0d = rint(cN);
+    if (!edges_fit(cN) || !limbs_fit(w, q)) {
+        const int64_t i0 = (int64_t)i0d;
+        double prev = edge_half_erf(i0 - R, c, Nd);
 #pragma unroll 1
+        for (int j = -R; j <= R; ++j) {
+            double next = edge_half_erf(i0 + j + 1, c, Nd);
+            double wt = next - prev;
+            prev = next;
+            double a = wt * w;
+            if (a != 0.0) lds_add_fxp(acc, N, cell0(i0 + j, nmask), fxp_from(a, q));
+        }
+        return;
+    }
+    double f[2 * R + 2];
+    gauss_edges<R>(c, i0d, Nd, 1.0 / Nd, f);
+    const int32_t i0 = (int32_t)(int64_t)i0d;
+#pragma unroll
     for (int j = -R; j <= R; ++j) {
-        double next = edge_half_erf(i0 + j + 1, c, Nd);
-        double wt = next - prev;
-        prev = next;
-        double a = wt * w;
-        if (a != 0.0) lds_add_fxp(acc, N, cell0(i0 + j, nmask), fxp_from(a, q));
+        if (j == -7 || j == 7) continue;  // both edges beyond 6: the weight is exactly 0
+        const double wt = f[j + R + 1] - f[j + R];
+        lds_add_contribution(acc, N, (i0 + j - 1) & nmask, wt * w, q);
     }
 }
 
