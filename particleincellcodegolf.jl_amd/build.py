@@ -32,6 +32,7 @@ SOURCES = ["kernels_1d.hip", "kernels_mixed.hip", "kernels_mixed_aux.hip", "kern
 # 103 scalar registers into vector lanes; without the hoisting the FP64
 # midpoint step (N = 4096, 3e6 particles) takes 1.00 in place of 1.03 ms.
 EXTRA_FLAGS = {"kernels_1d.hip": ["-mllvm", "-disable-machine-licm"],
+               "kernels_small.hip": ["-mllvm", "-disable-machine-licm"],
                "kernels_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
 
 

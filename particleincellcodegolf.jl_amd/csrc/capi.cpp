@@ -480,8 +480,8 @@ int pic_create_batch(pic_ctx** out, const pic_config* cfgs, int32_t n) {
     if ((rc = build_tables(c))) return fail(rc);
     if (c->ninst == 1 && small_eligible(c->hinst[0], c->scheme, c->precision, &c->small_K)) {
         c->small_ok = true;
-        if ((rc = dalloc(c, &c->small_gacc, 9 * (size_t)c->hinst[0].N))) return fail(rc);
-        if ((rc = dalloc(c, &c->small_bar, 4))) return fail(rc);
+        if ((rc = dalloc(c, &c->small_gacc, 9 * kSmallCopies * (size_t)c->hinst[0].N))) return fail(rc);
+        if ((rc = dalloc(c, &c->small_bar, kSmallBarWords))) return fail(rc);
     }
     *out = c;
     return PIC_OK;
@@ -791,15 +791,16 @@ static int run_small(pic_ctx* c, int64_t nsteps, double* diag, int32_t* sweeps) 
     a.bar = c->small_bar;
     a.K = (int32_t)c->small_K;
     a.spin_limit = 1u << 22;
-    HIPCHK(c, hipMemsetAsync(c->small_gacc, 0, 9 * sizeof(unsigned long long) * (size_t)a.I.N, c->stream));
-    HIPCHK(c, hipMemsetAsync(c->small_bar, 0, 4 * sizeof(uint32_t), c->stream));
+    HIPCHK(c, hipMemsetAsync(c->small_gacc, 0, 9 * kSmallCopies * sizeof(unsigned long long) * (size_t)a.I.N,
+                             c->stream));
+    HIPCHK(c, hipMemsetAsync(c->small_bar, 0, kSmallBarWords * sizeof(uint32_t), c->stream));
     HIPCHK(c, launch_small_run(a, c->scheme, c->stream));
-    uint32_t bar[4] = {0, 0, 0, 0};
-    HIPCHK(c, hipMemcpyAsync(bar, c->small_bar, sizeof bar, hipMemcpyDeviceToHost, c->stream));
+    uint32_t aborted = 0;
+    HIPCHK(c, hipMemcpyAsync(&aborted, c->small_bar + kSmallAbort, sizeof aborted, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     // the run moved the state past any charge a graph step primed
     c->primed = false;
-    if (bar[2]) {
+    if (aborted) {
         set_err(c, "pic_run: a grid barrier of the persistent run timed out (run state undefined)");
         return PIC_EHIP;
     }

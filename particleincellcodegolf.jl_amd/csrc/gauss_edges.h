@@ -262,6 +262,37 @@ PIC_HD void erf_inner(d2& c, d2& a, d2& b) {
     }
 }
 
+// erf(z) for |z| in [M, M+1] where M differs from lane to lane: every lane
+// evaluates every form and selects its own.
+PIC_HD double erf_any(double z, int M) {
+    typedef double d1 __attribute__((ext_vector_type(1)));
+    const double erx = 8.45062911510467529297e-01;
+    const double x = __builtin_fabs(z);
+    d1 P, Q, R, S, Rb, Sb;
+    erf_near1(d1(x), P, Q);
+    const double xe = M >= 1 ? x : 1.5;  // keeps the exponential form's operands in the range of div_normal
+    const d1 s = div_normal(d1(1.0), d1(xe * xe));
+    erf_RS_A(s, R, S);
+    erf_RS_B(s, Rb, Sb);
+    const bool far = hi32(xe) >= 0x4006DB6Eu;
+    const double r = erf_exponentials(d1(xe), far ? Rb : R, far ? Sb : S)[0];
+    const double w = z * z;
+    const double p = 1.28379167095512558561e-01 +
+                     w * (-3.25042107247001499370e-01 +
+                          w * (-2.84817495755985104766e-02 +
+                               w * (-5.77027029648944159157e-03 + w * -2.37630166566501626084e-05)));
+    const double q = 1.0 + w * (3.97917223959155352819e-01 +
+                                w * (6.50222499887672944485e-02 +
+                                     w * (5.08130628187576562776e-03 +
+                                          w * (1.32494738004321644526e-04 + w * -3.96022827877536812320e-06))));
+    const bool near1 = (M == 0 && hi32(x) >= 0x3feb0000u) || (M == 1 && hi32(x) < 0x3ff40000u);
+    const bool center = M == 0 && !near1;
+    const double y = div_normal(d1(near1 ? P[0] : center ? p : r), d1(near1 ? Q[0] : center ? q : xe))[0];
+    if (center) return z + z * (hi32(x) < 0x3e300000u ? 1.28379167095512586316e-01 : y);
+    const double e = near1 ? erx + y : hi32(x) >= 0x40180000u ? 1.0 : 1.0 - y;
+    return __builtin_copysign(e, z);
+}
+
 // f[j] = erf(z_j)/2 for z_j = ((i0 + (j - R - 1/2))/N - c)*N, j = 0..2R+1,
 // where i0 = rint(c*N) and |c*N| < 2^51: the edge arguments of the scripts
 // (src/GaussianFixedPointQuiet.jl:5), whose (i - 1/2) and, N being a power of
@@ -299,6 +330,14 @@ PIC_HD void gauss_edges(double c, double i0, double Nd, double iN, double (&f)[2
             if (j == R + 4 + t) f[R + 4 + t] = e;
         }
     }
+}
+
+// One edge of those, j in [0, 2R+1] (lanes of one particle hold one edge each;
+// any other j gives a value of no use).
+template <int R>
+PIC_HD double gauss_edge(double c, double i0, int j, double Nd, double iN) {
+    const double z = ((i0 + ((double)(j - R) - 0.5)) * iN - c) * Nd;
+    return erf_any(z, j <= R ? R - j : j - R - 1) * 0.5;
 }
 
 // A contribution |a| on the 2^-q grid as the three 43-bit limbs of

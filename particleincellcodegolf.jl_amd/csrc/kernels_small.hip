@@ -30,6 +30,7 @@
 #include "pic_internal.h"
 #include "solve1d.h"
 #include "stencil1d.h"
+#include "wave_ops.h"
 
 #pragma clang fp contract(off)
 
@@ -39,20 +40,18 @@ constexpr int kSmallThreads = kSolveThreads;  // threads per workgroup of both k
 constexpr int kSegLanes = 16;       // lanes per particle in k_small_gauss
 constexpr int kSegs = kSmallThreads / kSegLanes;
 
-// LDS layout shared by both kernels (doubles): the forward and the inverse
-// transform (re, im each), the previous field, reduction scratch, the field,
-// diagnostics partials, the solve's tables (stage twiddles of an N-point
-// transform as double2, then the 1/(2 pi k) factors), the u64 charge
-// counters (NGP: N counts; Gaussian: 3 N limbs), and (NGP) the exchange of
-// the upper half's velocities for the diagnostics tree.
-constexpr int kNgpXchg = (kSmallThreads / 2) * kSmallNgpSlots;
+// LDS layout shared by both kernels (doubles): the charge (bit-reversed), the
+// solve's permutation (re, im), the previous field, the field, reduction
+// scratch, diagnostics partials, the solve's tables (stage twiddles of an
+// N-point transform as double2, then the 1/(2 pi k) factors) and the u64
+// charge counters (NGP: N counts; Gaussian: 3 N limbs).
 __host__ __device__ constexpr int small_lds_doubles(int N) {
-    return 4 * N + 2 * N + kRedDoubles + 8 + 2 * N + (N / 2 + 1) + 3 * N;
+    return 5 * N + kRedDoubles + 8 + 2 * N + (N / 2 + 1) + 3 * N;
 }
-int small_lds_bytes(int N, bool ngp) { return 8 * (small_lds_doubles(N) + (ngp ? kNgpXchg : 0)); }
+int small_lds_bytes(int N) { return 8 * small_lds_doubles(N); }
 
 struct SmallLds {
-    double *re, *im, *bre, *bim, *Fl, *red, *Eld, *dp, *xi, *xchg;
+    double *re, *bre, *bim, *Fl, *red, *Eld, *dp, *xi;
     double2* tw;
     u64* acc;
 };
@@ -60,17 +59,15 @@ struct SmallLds {
 __device__ __forceinline__ SmallLds small_lds(double* sm, int N) {
     SmallLds L;
     L.re = sm;
-    L.im = sm + N;
-    L.bre = sm + 2 * N;
-    L.bim = sm + 3 * N;
-    L.Fl = sm + 4 * N;
-    L.red = L.Fl + N;
-    L.Eld = L.red + kRedDoubles;
-    L.dp = L.Eld + N;
+    L.bre = sm + N;
+    L.bim = sm + 2 * N;
+    L.Fl = sm + 3 * N;
+    L.Eld = sm + 4 * N;
+    L.red = sm + 5 * N;
+    L.dp = L.red + kRedDoubles;
     L.tw = reinterpret_cast<double2*>(L.dp + 8);
     L.xi = L.dp + 8 + 2 * N;
     L.acc = reinterpret_cast<u64*>(L.xi + N / 2 + 1);
-    L.xchg = reinterpret_cast<double*>(L.acc + 3 * N);
     return L;
 }
 
@@ -85,351 +82,388 @@ __device__ __forceinline__ void stage_tables(const SmallLds& L, const double2* _
 
 // ---------------------------------------------------------------------------
 // The solve in one wave.  Element i of an N-point (N <= 256) transform lives in
-// lane i % 64, slot i / 64 of wave 0.  A radix-2 stage with half-size h < 64
-// pairs lanes l and l ^ h (lane shuffles), with h >= 64 slots q and q + h/64
-// of one lane; every butterfly is the stage-by-stage transform's (operands
-// b = the upper element, a = the lower, t = b w, a + t and a - t; twiddle of
-// stage s at table entry 2^(s-1) - 1 + j, conjugated for the inverse), so
-// the result is that of the CPU restatement bit for bit.
+// lane i % 64, slot i / 64 < E of wave 0 (E = 1 up to N = 64).  A radix-2 stage
+// with half-size h < 64 pairs lanes l and l ^ h, with h >= 64 slots q and
+// q + h/64 of one lane; every butterfly is the stage-by-stage transform's
+// (operands b = the upper element, a = the lower, t = b w, a + t and a - t;
+// twiddle of stage s at table entry 2^(s-1) - 1 + j, conjugated for the
+// inverse), so the result is that of the CPU restatement bit for bit.
+//
+// One wave with six dependent stages each way is a latency chain: the lane
+// exchanges stay in registers (wave_ops.h), a lane's twiddles and 1/(2 pi k)
+// factors too, and the three norms of the test share their trees' steps.  At
+// N = 64 the solve with its test took 12800 cycles with shuffles through LDS.
 // ---------------------------------------------------------------------------
-constexpr int kWaveSlots = kSmallMaxN / 64;
 
-__device__ __forceinline__ void wave_radix2(double (&re)[kWaveSlots], double (&im)[kWaveSlots],
-                                            const double2* __restrict__ tw, int N, int log2N, bool inverse) {
+// What a lane of wave 0 keeps of the tables.
+template <int E>
+struct WaveTables {
+    double2 w[6];  // its twiddle of the stages with h < 64
+    double xt[E];  // 1/(2 pi k') of its modes
+};
+
+template <int E>
+__device__ __forceinline__ void load_wave_tables(WaveTables<E>& W, const SmallLds& L, int N) {
     const int l = threadIdx.x & 63;
-    const int E = N >= 64 ? N >> 6 : 1;
-    for (int st = 1; st <= log2N; ++st) {
-        const int h = 1 << (st - 1);
-        if (h < 64) {
-            const bool lower = (l & h) == 0;
-            const double2 w = tw[h - 1 + (l & (h - 1))];
-            const double wr = w.x, wi = inverse ? -w.y : w.y;
 #pragma unroll
-            for (int q = 0; q < kWaveSlots; ++q) {
-                if (q >= E) break;
-                const double pr = __shfl_xor(re[q], h, 64), pi = __shfl_xor(im[q], h, 64);
-                const double br = lower ? pr : re[q], bi = lower ? pi : im[q];
-                const double ar = lower ? re[q] : pr, ai = lower ? im[q] : pi;
-                const double tr = br * wr - bi * wi;
-                const double tq = br * wi + bi * wr;
-                re[q] = lower ? ar + tr : ar - tr;
-                im[q] = lower ? ai + tq : ai - tq;
-            }
-        } else {
-            const int hs = h >> 6;
+    for (int s = 0; s < 6; ++s) {
+        const int h = 1 << s;
+        W.w[s] = h < N ? L.tw[h - 1 + (l & (h - 1))] : double2{0.0, 0.0};
+    }
 #pragma unroll
-            for (int q = 0; q < kWaveSlots; ++q) {
-                if ((q & hs) || q + hs >= E) continue;
-                const double2 w = tw[h - 1 + ((q * 64 + l) & (h - 1))];
-                const double wr = w.x, wi = inverse ? -w.y : w.y;
+    for (int q = 0; q < E; ++q) {
+        const int m = q * 64 + l;
+        W.xt[q] = m >= N ? 0.0 : m == 0 ? L.xi[1] : (m <= N / 2 ? L.xi[m] : -L.xi[N - m]);
+    }
+}
+
+// x with its sign flipped where `upper`
+__device__ __forceinline__ double flip_if(bool upper, double x) {
+    return __longlong_as_double(__double_as_longlong(x) ^ (upper ? (long long)0x8000000000000000ull : 0ll));
+}
+
+template <int E, int H>
+__device__ __forceinline__ void wave_stage(double (&re)[E], double (&im)[E], double wr, double wi) {
+    const bool upper = (threadIdx.x & H) != 0;
 #pragma unroll
-                for (int qq = 0; qq < kWaveSlots; ++qq) {
-                    if (qq != q + hs) continue;
-                    const double br = re[qq], bi = im[qq];
-                    const double tr = br * wr - bi * wi;
-                    const double tq = br * wi + bi * wr;
-                    const double ar = re[q], ai = im[q];
-                    re[q] = ar + tr;
-                    im[q] = ai + tq;
-                    re[qq] = ar - tr;
-                    im[qq] = ai - tq;
-                }
-            }
+    for (int q = 0; q < E; ++q) {
+        double ar, ai, br, bi;
+        lane_pair<H>(re[q], ar, br);
+        lane_pair<H>(im[q], ai, bi);
+        const double tr = br * wr - bi * wi;
+        const double tq = br * wi + bi * wr;
+        re[q] = ar + flip_if(upper, tr);  // a - t is a + (-t)
+        im[q] = ai + flip_if(upper, tq);
+    }
+}
+
+template <int E>
+__device__ __forceinline__ void wave_radix2(double (&re)[E], double (&im)[E], const WaveTables<E>& W,
+                                            const double2* __restrict__ tw, int N, bool inverse) {
+    auto wi = [&](int s) { return inverse ? -W.w[s].y : W.w[s].y; };
+    if (N > 1) wave_stage<E, 1>(re, im, W.w[0].x, wi(0));
+    if (N > 2) wave_stage<E, 2>(re, im, W.w[1].x, wi(1));
+    if (N > 4) wave_stage<E, 4>(re, im, W.w[2].x, wi(2));
+    if (N > 8) wave_stage<E, 8>(re, im, W.w[3].x, wi(3));
+    if (N > 16) wave_stage<E, 16>(re, im, W.w[4].x, wi(4));
+    if (N > 32) wave_stage<E, 32>(re, im, W.w[5].x, wi(5));
+    const int l = threadIdx.x & 63;
+#pragma unroll
+    for (int hs = 1; hs < E; hs <<= 1) {
+        const int h = hs * 64;
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            if (q & hs) continue;
+            const double2 w = tw[h - 1 + ((q * 64 + l) & (h - 1))];
+            const double wr = w.x, wq = inverse ? -w.y : w.y;
+            const double br = re[q + hs], bi = im[q + hs];
+            const double tr = br * wr - bi * wq;
+            const double tq = br * wq + bi * wr;
+            const double ar = re[q], ai = im[q];
+            re[q] = ar + tr;
+            im[q] = ai + tq;
+            re[q + hs] = ar - tr;
+            im[q + hs] = ai - tq;
         }
     }
 }
 
 // The canonical reduction tree (tree256 over lanes t < 256 that each fold the
-// elements t, t + 256, ... in order from +0.0) over the N values x of wave 0
-// (N <= 256 here; the loop also folds slot u + 4, which N = 512 would fill):
-// tree lane t = l + 64u folds slot u of lane l, the two
-// halving steps combine (u, u + 2) and then (0, 1) in lane l, and the last
-// six steps are tree256's own shuffles.  MAX: the NaN-propagating maximum.
-// Every value is >= 0 (squares, magnitudes, flags), so folding +0.0 for a
-// missing element leaves a sum or maximum unchanged.  Lane 0's result is
-// returned to every lane.
-template <bool MAX>
-__device__ __forceinline__ double wave_canon(const double (&x)[kWaveSlots], int N) {
-    auto op = [](double a, double b) { return MAX ? nanmax(a, b) : a + b; };
-    const int l = threadIdx.x & 63;
-    double P[4];
+// elements t, t + 256, ... from +0.0) of K arrays of N <= 256 values in wave 0:
+// tree lane t = l + 64u folds slot u of lane l, the two halving steps combine
+// (u, u + 2) and then (0, 1) in lane l, and the last six steps are wave_tree's.
+// op(k, a, b): array k's sum or NaN-propagating maximum.  Every value is >= 0
+// (squares, magnitudes, flags), so folding +0.0 for a missing element leaves a
+// sum or maximum unchanged.
+template <int K, int E, typename F>
+__device__ __forceinline__ void wave_canon(double (&r)[K], const double (&x)[K][E], F&& op) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        P[u] = 0.0;
+    for (int k = 0; k < K; ++k) {
+        double P[4];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const int q = u + 4 * k;
-            if (q < kWaveSlots && q * 64 + l < N) P[u] = op(P[u], x[q]);
-        }
+        for (int u = 0; u < 4; ++u) P[u] = u < E ? op(k, 0.0, x[k][u < E ? u : 0]) : 0.0;
+        r[k] = E > 2 ? op(k, op(k, P[0], P[2]), op(k, P[1], P[3])) : E > 1 ? op(k, P[0], P[1]) : P[0];
     }
-    double r = op(op(P[0], P[2]), op(P[1], P[3]));
-#pragma unroll
-    for (int h = 32; h > 0; h >>= 1) r = op(r, __shfl_down(r, h, 64));
-    return __shfl(r, 0, 64);
+    wave_tree<K>(r, op);
 }
 
-// The solve of the charge staged in re/im (bit-reversed), in wave 0:
+// In wave 0: the solve of the charge staged in L.re (bit-reversed),
 // E = real(ifft((xi = fft(rho) ./ ik; xi[1] *= 0; xi))) into Eld, with ik and
 // Julia's division by (0, 2 pi k') as in k_solve; with TEST also the
 // convergence test isapprox(Fl, E) of the midpoint loop, with block_isapprox's
-// norms and decisions (Fl then takes E).  Returns the test's result; emax
-// gets max |E|.  Every thread of the block calls it.
-template <bool TEST>
-__device__ __forceinline__ bool small_solve(const SmallLds& L, int N, int log2N, double rtol, double& emax) {
-    if (threadIdx.x < 64) {
-        const int l = threadIdx.x;
-        double re[kWaveSlots], im[kWaveSlots];
+// norms and decisions (Fl then takes E).  red gets max |E|, the test's result
+// and the canonical sum of E^2.
+template <bool TEST, int E>
+__device__ __forceinline__ void wave_solve(const SmallLds& L, const WaveTables<E>& W, int N, int log2N, double rtol) {
+    const int l = threadIdx.x;
+    double re[E], im[E];
 #pragma unroll
-        for (int q = 0; q < kWaveSlots; ++q) {
-            const int i = q * 64 + l;
-            re[q] = i < N ? L.re[i] : 0.0;
-            im[q] = i < N ? L.im[i] : 0.0;
-        }
-        wave_radix2(re, im, L.tw, N, log2N, false);
-#pragma unroll
-        for (int q = 0; q < kWaveSlots; ++q) {
-            const int m = q * 64 + l;
-            if (m >= N) continue;
-            const double t = m == 0 ? L.xi[1] : (m <= N / 2 ? L.xi[m] : -L.xi[N - m]);
-            double a = im[q] * t;
-            double b = -(re[q] * t);
-            if (m == 0) {
-                a = a * 0.0;
-                b = b * 0.0;
-            }
-            const int p = (int)brev((uint32_t)m, log2N);
-            L.bre[p] = a;
-            L.bim[p] = b;
-        }
-        // the permutation stays inside the wave: LDS operations of one wave
-        // complete in order; the fences keep the compiler from moving them
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int q = 0; q < kWaveSlots; ++q) {
-            const int i = q * 64 + l;
-            re[q] = i < N ? L.bre[i] : 0.0;
-            im[q] = i < N ? L.bim[i] : 0.0;
-        }
-        wave_radix2(re, im, L.tw, N, log2N, true);
-        const double scale = 1.0 / (double)N;
-        double e[kWaveSlots];
-#pragma unroll
-        for (int q = 0; q < kWaveSlots; ++q) {
-            const int i = q * 64 + l;
-            e[q] = re[q] * scale;
-            if (i < N) L.Eld[i] = e[q];
-        }
-        bool conv = false;
-        double me;
-        if (TEST) {
-            double f[kWaveSlots], x[kWaveSlots];
-#pragma unroll
-            for (int q = 0; q < kWaveSlots; ++q) {
-                const int i = q * 64 + l;
-                f[q] = i < N ? L.Fl[i] : 0.0;
-            }
-            // the three norms of block_norms3: d = F - E, F, E
-            double m3[3], s3[3];
-#pragma unroll
-            for (int v = 0; v < 3; ++v) {
-#pragma unroll
-                for (int q = 0; q < kWaveSlots; ++q) {
-                    const double xv = v == 0 ? f[q] - e[q] : (v == 1 ? f[q] : e[q]);
-                    x[q] = fabs(xv);
-                }
-                m3[v] = wave_canon<true>(x, N);
-#pragma unroll
-                for (int q = 0; q < kWaveSlots; ++q) {
-                    const double xv = v == 0 ? f[q] - e[q] : (v == 1 ? f[q] : e[q]);
-                    x[q] = xv * xv;
-                }
-                s3[v] = wave_canon<false>(x, N);
-            }
-            double nrm[3];
-#pragma unroll
-            for (int v = 0; v < 3; ++v) {
-                const bool direct = m3[v] == 0.0 || isinf(m3[v]);
-                const bool scaled = !direct && !(isfinite((double)N * m3[v] * m3[v]) && m3[v] * m3[v] != 0.0);
-                if (scaled) {
-#pragma unroll
-                    for (int q = 0; q < kWaveSlots; ++q) {
-                        const double xv = v == 0 ? f[q] - e[q] : (v == 1 ? f[q] : e[q]);
-                        const double y = fabs(xv) / m3[v];
-                        x[q] = y * y;
-                    }
-                    s3[v] = wave_canon<false>(x, N);
-                }
-                nrm[v] = direct ? m3[v] : (scaled ? m3[v] * sqrt(s3[v]) : sqrt(s3[v]));
-            }
-            me = m3[2];
-            const double dn = nrm[0], nf = nrm[1], ne = nrm[2];
-            if (isfinite(dn)) {
-                double mx = nf > ne ? nf : ne;
-                if (nf != nf || ne != ne) mx = __longlong_as_double(0x7ff8000000000000LL);
-                const double tol = rtol * mx;
-                double lim = 0.0 > tol ? 0.0 : tol;
-                if (tol != tol) lim = tol;
-                conv = dn <= lim;
-            } else {
-#pragma unroll
-                for (int q = 0; q < kWaveSlots; ++q) {
-                    const double a = f[q], b = e[q];
-                    bool good = a == b;
-                    if (!good && isfinite(a) && isfinite(b)) {
-                        const double ma = fabs(a) > fabs(b) ? fabs(a) : fabs(b);
-                        const double t = rtol * ma;
-                        good = fabs(a - b) <= (0.0 > t ? 0.0 : t);
-                    }
-                    x[q] = good ? 0.0 : 1.0;
-                }
-                conv = wave_canon<true>(x, N) == 0.0;
-            }
-#pragma unroll
-            for (int q = 0; q < kWaveSlots; ++q) {
-                const int i = q * 64 + l;
-                if (i < N) L.Fl[i] = e[q];
-            }
-        } else {
-            double x[kWaveSlots];
-#pragma unroll
-            for (int q = 0; q < kWaveSlots; ++q) x[q] = fabs(e[q]);
-            me = wave_canon<true>(x, N);
-        }
-        if (l == 0) {
-            L.red[0] = me;
-            L.red[1] = conv ? 1.0 : 0.0;
-        }
+    for (int q = 0; q < E; ++q) {
+        const int i = q * 64 + l;
+        re[q] = i < N ? L.re[i] : 0.0;
+        im[q] = 0.0;
     }
-    __syncthreads();
-    emax = L.red[0];
-    const bool conv = L.red[1] != 0.0;
-    __syncthreads();
-    return conv;
+    double f[E];
+    if (TEST)
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            f[q] = i < N ? L.Fl[i] : 0.0;
+        }
+    wave_radix2<E>(re, im, W, L.tw, N, false);
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int m = q * 64 + l;
+        if (m >= N) continue;
+        double a = im[q] * W.xt[q];
+        double b = -(re[q] * W.xt[q]);
+        if (m == 0) {
+            a = a * 0.0;
+            b = b * 0.0;
+        }
+        const int p = (int)brev((uint32_t)m, log2N);
+        L.bre[p] = a;
+        L.bim[p] = b;
+    }
+    // the permutation stays inside the wave: LDS operations of one wave
+    // complete in order; the fences keep the compiler from moving them
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int i = q * 64 + l;
+        re[q] = i < N ? L.bre[i] : 0.0;
+        im[q] = i < N ? L.bim[i] : 0.0;
+    }
+    wave_radix2<E>(re, im, W, L.tw, N, true);
+    const double scale = 1.0 / (double)N;
+    double e[E];
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int i = q * 64 + l;
+        e[q] = i < N ? re[q] * scale : 0.0;
+        if (i < N) L.Eld[i] = e[q];
+    }
+    bool conv = false;
+    double me, se;
+    if (TEST) {
+        // the three norms of block_norms3: d = F - E, F, E; maxima 0..2, sums of squares 3..5
+        double x[6][E], r[6];
+        auto op = [](int k, double a, double b) { return k < 3 ? nanmax(a, b) : a + b; };
+        auto val = [&](int v, int q) { return v == 0 ? f[q] - e[q] : (v == 1 ? f[q] : e[q]); };
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const double xv = val(v, q);
+                x[v][q] = fabs(xv);
+                x[3 + v][q] = xv * xv;
+            }
+        wave_canon<6, E>(r, x, op);
+        me = r[2];
+        se = r[5];
+        double nrm[3];
+#pragma unroll
+        for (int v = 0; v < 3; ++v) {
+            const double m = r[v];
+            const bool direct = m == 0.0 || isinf(m);
+            const bool scaled = !direct && !(isfinite((double)N * m * m) && m * m != 0.0);
+            double s = r[3 + v];
+            if (scaled) {
+                double y[1][E], t[1];
+#pragma unroll
+                for (int q = 0; q < E; ++q) {
+                    const double z = q * 64 + l < N ? fabs(val(v, q)) / m : 0.0;
+                    y[0][q] = z * z;
+                }
+                wave_canon<1, E>(t, y, [](int, double a, double b) { return a + b; });
+                s = t[0];
+            }
+            nrm[v] = direct ? m : (scaled ? m * sqrt(s) : sqrt(s));
+        }
+        const double dn = nrm[0], nf = nrm[1], ne = nrm[2];
+        if (isfinite(dn)) {
+            double mx = nf > ne ? nf : ne;
+            if (nf != nf || ne != ne) mx = __longlong_as_double(0x7ff8000000000000LL);
+            const double tol = rtol * mx;
+            double lim = 0.0 > tol ? 0.0 : tol;
+            if (tol != tol) lim = tol;
+            conv = dn <= lim;
+        } else {
+            double y[1][E], t[1];
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const double a = f[q], b = e[q];
+                bool good = a == b;
+                if (!good && isfinite(a) && isfinite(b)) {
+                    const double ma = fabs(a) > fabs(b) ? fabs(a) : fabs(b);
+                    const double tl = rtol * ma;
+                    good = fabs(a - b) <= (0.0 > tl ? 0.0 : tl);
+                }
+                y[0][q] = good ? 0.0 : 1.0;
+            }
+            wave_canon<1, E>(t, y, [](int, double a, double b) { return nanmax(a, b); });
+            conv = t[0] == 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            if (i < N) L.Fl[i] = e[q];
+        }
+    } else {
+        double x[2][E], r[2];
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            x[0][q] = fabs(e[q]);
+            x[1][q] = e[q] * e[q];
+        }
+        wave_canon<2, E>(r, x, [](int k, double a, double b) { return k < 1 ? nanmax(a, b) : a + b; });
+        me = r[0];
+        se = r[1];
+    }
+    if (l == 0) {
+        L.red[0] = me;
+        L.red[1] = conv ? 1.0 : 0.0;
+        L.red[2] = se;
+    }
 }
 
-// D[t,1:4] of one step from the field in Eld and the chunk partials in dp
-// (src/GaussianFixedPointQuiet.jl:11,13), as k_diag_final writes it.
-__device__ __forceinline__ void small_diag_row(const SmallLds& L, const InstDesc& I, int64_t nchunks,
+// D[t,1:4] of one step from the canonical sum of E^2 and the chunk partials in
+// dp (src/GaussianFixedPointQuiet.jl:11,13), as k_diag_final writes it: the
+// tree over at most four partials is (p0 + p2) + (p1 + p3) with +0.0 for the
+// missing ones, each folded from +0.0.  One thread calls it.
+__device__ __forceinline__ void small_diag_row(const SmallLds& L, const InstDesc& I, double se, int nch,
                                                double* __restrict__ row4, int32_t* __restrict__ sweeps,
                                                int32_t nsweeps) {
-    double se, sv, sp;
-    diag_sums(L.red, L.Eld, I.N, L.dp, nchunks, se, sv, sp);
-    if (threadIdx.x == 0) {
-        const double d1 = (se / (double)I.N) / 2.0;
-        const double d2 = ((sv * I.W) / (double)I.P) / 2.0;
-        const double d3 = d1 + d2;
-        const double s = 2.0 / I.W;
-        row4[0] = d1 * s;
-        row4[1] = d2 * s;
-        row4[2] = d3 * s;
-        row4[3] = sp;
-        *sweeps = nsweeps;
-    }
+    double p[2][4];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) p[k][c] = c < nch ? 0.0 + L.dp[2 * c + k] : 0.0;
+    const double sv = (p[0][0] + p[0][2]) + (p[0][1] + p[0][3]), sp = (p[1][0] + p[1][2]) + (p[1][1] + p[1][3]);
+    const double d1 = (se / (double)I.N) / 2.0;
+    const double d2 = ((sv * I.W) / (double)I.P) / 2.0;
+    const double d3 = d1 + d2;
+    const double s = 2.0 / I.W;
+    row4[0] = d1 * s;
+    row4[1] = d2 * s;
+    row4[2] = d3 * s;
+    row4[3] = sp;
+    *sweeps = nsweeps;
 }
 
+// v/P as the reference divides it: by the exact reciprocal where P is a power
+// of two
+struct DivP {
+    double P, rP;
+    bool pow2;
+    __device__ __forceinline__ explicit DivP(int64_t n) : P((double)n), rP(1.0 / (double)n), pow2((n & (n - 1)) == 0) {}
+    __device__ __forceinline__ double operator()(double v) const { return pow2 ? v * rP : v / P; }
+};
+
 // ---------------------------------------------------------------------------
-// NGP leapfrog (src/NGPFourier.jl:4-6), one workgroup, J particles per thread.
+// NGP leapfrog (src/NGPFourier.jl:4-6), one workgroup.  Thread t holds lane
+// t % 256 of diagnostics chunk t / 256 (particles 4096 (t / 256) + t % 256 +
+// 256 i, i < 16), so the sums of a chunk's lanes need no exchange; their trees
+// run in waves 1 and 2 beside the next step's solve in wave 0.
 // ---------------------------------------------------------------------------
-template <int JMAX>
+template <int E>
 __global__ void __launch_bounds__(kSmallThreads)
 k_small_ngp(SmallRun a) {
     extern __shared__ double sm[];
+    constexpr int J = kSmallNgpSlots;
+    static_assert(J * kTreeLanes == kTreeChunk && kSmallThreads == 2 * kTreeLanes, "one lane of one chunk per thread");
     const InstDesc I = a.I;
     InstState S = *a.st;
     const int N = I.N, log2N = I.log2N;
     const SmallLds L = small_lds(sm, N);
     const int t = threadIdx.x;
     const int64_t P = I.P;
-    const double Nd = (double)N, dt = I.dt, Pd = (double)P;
+    const double Nd = (double)N, dt = I.dt;
+    const DivP divP(P);
     const int32_t nmask = I.nmask;
     const int par0 = S.step & 1;
     const double* X = par0 ? a.X1 : a.X0;
     const double* V = par0 ? a.V1 : a.V0;
-    // particle t + 512 j
-    double x[JMAX], v[JMAX];
-    bool has[JMAX];
+    double x[J], v[J];
+    bool has[J];
+    const int64_t p0 = (int64_t)(t / kTreeLanes) * kTreeChunk + (t % kTreeLanes);
 #pragma unroll
-    for (int j = 0; j < JMAX; ++j) {
-        const int64_t p = t + (int64_t)kSmallThreads * j;
+    for (int j = 0; j < J; ++j) {
+        const int64_t p = p0 + (int64_t)kTreeLanes * j;
         has[j] = p < P;
         x[j] = has[j] ? X[p] : 0.0;
         v[j] = has[j] ? V[p] : 0.0;
     }
     stage_tables(L, a.tw, N);
+    WaveTables<E> W;
+    load_wave_tables<E>(W, L, N);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(L.acc);
+    for (int c = t; c < N; c += kSmallThreads) cnt[c] = 0;
     const u128 one = fxp_from(I.w, I.q);
-    const int64_t nch = (P + kTreeChunk - 1) / kTreeChunk;
-    constexpr int kPerChunk = kTreeChunk / kSmallThreads;  // slots j of one diagnostics chunk
+    const int nch = (int)((P + kTreeChunk - 1) / kTreeChunk);
+    double se = 0.0;  // of the step whose row is still to be written
     bool bad = false;
+    __syncthreads();
+    // the trees of chunk c's lane sums (L.red + 16 + 512 k + 256 c) into dp
+    auto trees = [&](int c) {
+        const int l = t & 63;
+        double r[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const double* q = L.red + 16 + 512 * k + kTreeLanes * c + l;
+            r[k] = (q[0] + q[128]) + (q[64] + q[192]);
+        }
+        wave_tree<2>(r, [](int, double x1, double x2) { return x1 + x2; });
+        if (l == 0) {
+            L.dp[2 * c] = r[0];
+            L.dp[2 * c + 1] = r[1];
+        }
+    };
     for (int64_t s = 0; s < a.nsteps; ++s) {
-        for (int c = t; c < N; c += kSmallThreads) L.acc[c] = 0;
-        __syncthreads();
         // u(); n[f(j)] += w (the count; times w exactly below)
 #pragma unroll
-        for (int j = 0; j < JMAX; ++j)
+        for (int j = 0; j < J; ++j)
             if (has[j]) {
                 x[j] = jl_mod1f(x[j] + (v[j] / 2.0) * dt);
-                atomicAdd(&L.acc[ngp_cell(x[j], Nd, nmask)], 1ull);
+                atomicAdd(&cnt[ngp_cell(x[j], Nd, nmask)], 1u);
             }
         __syncthreads();
         for (int c = t; c < N; c += kSmallThreads) {
-            const int b = (int)brev((uint32_t)c, log2N);
-            L.re[b] = fxp_to((u128)L.acc[c] * one, I.q);
-            L.im[b] = 0.0;
+            L.re[(int)brev((uint32_t)c, log2N)] = fxp_to((u128)cnt[c] * one, I.q);
+            cnt[c] = 0;
         }
         __syncthreads();
-        double emax;
-        small_solve<false>(L, N, log2N, 0.0, emax);
-        bad = bad || !isfinite(emax);
-        // u(); v += E[f.(x)]*dt
+        if (t < 64) wave_solve<false, E>(L, W, N, log2N, 0.0);
+        else if (s > 0 && t < 64 * (1 + nch)) trees((t >> 6) - 1);
+        __syncthreads();
+        bad = bad || !isfinite(L.red[0]);
+        if (s > 0 && t == kSmallThreads - 1) small_diag_row(L, I, se, nch, a.diag + 4 * (s - 1), a.sweeps + s - 1, 1);
+        se = L.red[2];
+        // u(); v += E[f.(x)]*dt; the lane's sums of v^2 and v/P in order
+        double s2 = 0.0, s1 = 0.0;
 #pragma unroll
-        for (int j = 0; j < JMAX; ++j)
+        for (int j = 0; j < J; ++j)
             if (has[j]) {
                 x[j] = jl_mod1f(x[j] + (v[j] / 2.0) * dt);
                 v[j] = v[j] + L.Eld[ngp_cell(x[j], Nd, nmask)] * dt;
+                s2 = s2 + v[j] * v[j];
+                s1 = s1 + divP(v[j]);
             }
-        // chunk partials of v^2 and v/P.  Lane l < 256 of chunk c sums particles
-        // 4096 c + l + 256 i, i = 0..15, in order: those of thread l (i even,
-        // slot 8c + i/2) and of thread l + 256 (i odd), whose values come
-        // through LDS.
-        if (t >= kTreeLanes)
-#pragma unroll
-            for (int j = 0; j < JMAX; ++j) L.xchg[(t - kTreeLanes) * JMAX + j] = v[j];
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < JMAX / kPerChunk; ++c) {
-            if (c < nch) {
-                double s2 = 0.0, s1 = 0.0, z = 0.0;
-                if (t < kTreeLanes) {
-#pragma unroll
-                    for (int i = 0; i < kTreeChunk / kTreeLanes; ++i) {
-                        const int j = kPerChunk * c + i / 2;
-                        const int64_t p = (int64_t)kTreeChunk * c + t + (int64_t)kTreeLanes * i;
-                        if (p < P) {
-                            const double vv = (i & 1) ? L.xchg[t * JMAX + j] : v[j];
-                            s2 = s2 + vv * vv;
-                            s1 = s1 + vv / Pd;
-                        }
-                    }
-                }
-                tree256x3<false>(L.red, s2, s1, z);
-                if (t == 0) {
-                    L.dp[2 * c] = s2;
-                    L.dp[2 * c + 1] = s1;
-                }
-            }
-        }
-        __syncthreads();
-        small_diag_row(L, I, nch, a.diag + 4 * s, a.sweeps + s, 1);
-        __syncthreads();
+        L.red[16 + t] = s2;
+        L.red[16 + 512 + t] = s1;
     }
+    __syncthreads();
+    if (a.nsteps > 0 && t < 64 * nch) trees(t >> 6);
+    __syncthreads();
+    if (a.nsteps > 0 && t == 0) small_diag_row(L, I, se, nch, a.diag + 4 * (a.nsteps - 1), a.sweeps + a.nsteps - 1, 1);
     const int parN = (int)((S.step + a.nsteps) & 1);
     double* Xo = parN ? a.X1 : a.X0;
     double* Vo = parN ? a.V1 : a.V0;
 #pragma unroll
-    for (int j = 0; j < JMAX; ++j) {
-        const int64_t p = t + (int64_t)kSmallThreads * j;
+    for (int j = 0; j < J; ++j) {
+        const int64_t p = p0 + (int64_t)kTreeLanes * j;
         if (has[j]) {
             Xo[p] = x[j];
             Vo[p] = v[j];
@@ -446,37 +480,42 @@ k_small_ngp(SmallRun a) {
 }
 
 // ---------------------------------------------------------------------------
-// Grid barrier of k_small_gauss: a counter and a generation word, agent-scope
-// release/acquire (the pattern of a cooperative grid sync).  Every wait is
-// bounded: past spin_limit polls, or once another workgroup has given up, the
-// barrier reports failure and the caller leaves the kernel.
+// Grid barrier of k_small_gauss.  Each workgroup has a word of its own, which
+// takes the generation it arrived in (agent-scope release); the first wave of
+// every workgroup polls all of them, 64 to a load, until none is behind, then
+// acquires.  A shared counter instead made the arrivals queue: with the charge's
+// adds (below) the barrier took 19300 cycles at 65 workgroups and 4400 at two.
+// Every wait is bounded: past spin_limit polls, or once another workgroup has
+// given up (word kSmallAbort), the barrier reports failure and the caller
+// leaves the kernel.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ bool grid_barrier(uint32_t* bar, uint32_t nblocks, uint32_t& gen, uint32_t spin_limit,
+__device__ __forceinline__ bool grid_barrier(uint32_t* bar, int nblocks, uint32_t& gen, uint32_t spin_limit,
                                              int32_t* okflag) {
     __syncthreads();
-    if (threadIdx.x == 0) {
+    ++gen;
+    if (threadIdx.x < 64) {
+        if (threadIdx.x == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            __hip_atomic_store(&bar[blockIdx.x], gen, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
         int32_t ok = 1;
-        __threadfence();
-        const uint32_t arrived = __hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (arrived == nblocks - 1) {
-            __hip_atomic_store(&bar[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&bar[1], gen + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            uint32_t n = 0;
-            while (__hip_atomic_load(&bar[1], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == gen) {
-                if (++n > spin_limit ||
-                    __hip_atomic_load(&bar[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                    ok = 0;
-                    __hip_atomic_store(&bar[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
+        uint32_t n = 0;
+        for (;;) {
+            bool behind = false;
+            for (int b = threadIdx.x; b < nblocks; b += 64)
+                behind |= (int32_t)(__hip_atomic_load(&bar[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - gen) < 0;
+            if (__ballot(behind) == 0) break;
+            if (++n > spin_limit ||
+                __hip_atomic_load(&bar[kSmallAbort], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+                ok = 0;
+                if (threadIdx.x == 0)
+                    __hip_atomic_store(&bar[kSmallAbort], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
             }
         }
-        __threadfence();
-        *okflag = ok;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (threadIdx.x == 0) *okflag = ok;
     }
-    ++gen;
     __syncthreads();
     return *okflag != 0;
 }
@@ -492,41 +531,58 @@ __device__ __forceinline__ void st_agent(u64* p, u64 v) {
 // (src/GaussianFixedPointQuiet.jl:5); lane e of a particle's 16 holds it, and
 // weight e = f_{e+1} - f_e comes from the next lane.
 template <int R>
-__device__ __forceinline__ double seg_weight(int64_t i0, int e, double c, double Nd) {
-    const double f = edge_half_erf(i0 - R + e, c, Nd);
-    const double fn = __shfl_down(f, 1, kSegLanes);
-    return fn - f;
+__device__ __forceinline__ double seg_weight(double c, double Nd, double iN, int e, int32_t& cell0_, int32_t nmask) {
+    const double cN = c * Nd, i0 = rint(cN);
+    double f;
+    if (edges_fit(cN)) {
+        f = gauss_edge<R>(c, i0, e, Nd, iN);
+        cell0_ = ((int32_t)(int64_t)i0 - R - 1) & nmask;
+    } else {
+        f = edge_half_erf((int64_t)i0 - R + e, c, Nd);
+        cell0_ = cell0((int64_t)i0 - R, nmask);
+    }
+    return dpp_f64<0x101>(f, f) - f;  // the next lane's edge (lane 15 has none and no weight)
 }
 
 // sum(k -> E[k[1]]*k[2], d(c)): the products on lanes 0..2R, folded left in
-// cell order by every lane of the particle.
+// cell order by every lane of the particle (a row of the wave).
 template <int R>
-__device__ __forceinline__ double seg_gather(const double* __restrict__ Eld, double c, double Nd, int32_t nmask,
-                                             int e) {
-    const int64_t i0 = (int64_t)rint(c * Nd);
-    const double wt = seg_weight<R>(i0, e, c, Nd);
-    const double term = Eld[cell0(i0 - R + e, nmask)] * wt;
-    double S = __shfl(term, 0, kSegLanes);
-#pragma unroll
-    for (int q = 1; q <= 2 * R; ++q) S = S + __shfl(term, q, kSegLanes);
+__device__ __forceinline__ double seg_gather(const double* __restrict__ Eld, double c, double Nd, double iN,
+                                             int32_t nmask, int e) {
+    int32_t first;
+    const double wt = seg_weight<R>(c, Nd, iN, e, first, nmask);
+    const double term = Eld[(first + e) & nmask] * wt;
+    double S = dpp_f64<0x150>(term, term);  // row_newbcast: lane q of the row
+#define PIC_FOLD(q) S = S + dpp_f64<0x150 + q>(term, term)
+    PIC_FOLD(1); PIC_FOLD(2); PIC_FOLD(3); PIC_FOLD(4); PIC_FOLD(5); PIC_FOLD(6); PIC_FOLD(7); PIC_FOLD(8);
+    PIC_FOLD(9); PIC_FOLD(10); PIC_FOLD(11); PIC_FOLD(12);
+    if constexpr (R == 7) {
+        PIC_FOLD(13); PIC_FOLD(14);
+    }
+#undef PIC_FOLD
     return S;
 }
 
 // r[k[1]] += k[2]*w: lane e <= 2R adds cell i0 - R + e in exact limbs.
 template <int R>
-__device__ __forceinline__ void seg_deposit(u64* __restrict__ acc, int32_t N, double c, double Nd, int32_t nmask,
-                                            double w, int q, int e) {
-    const int64_t i0 = (int64_t)rint(c * Nd);
-    const double wt = seg_weight<R>(i0, e, c, Nd);
-    const double a = wt * w;
-    if (e <= 2 * R && a != 0.0) lds_add_fxp(acc, N, cell0(i0 - R + e, nmask), fxp_from(a, q));
+__device__ __forceinline__ void seg_deposit(u64* __restrict__ acc, int32_t N, double c, double Nd, double iN,
+                                            int32_t nmask, double w, int q, bool fit, int e) {
+    int32_t first;
+    const double a = seg_weight<R>(c, Nd, iN, e, first, nmask) * w;
+    if (e > 2 * R || !(a != 0.0)) return;
+    const int32_t cell = (first + e) & nmask;
+    if (fit) lds_add_contribution(acc, N, cell, a, q);
+    else lds_add_fxp(acc, N, cell, fxp_from(a, q));
 }
 
-// Adds this workgroup's LDS limbs into the device accumulator (re-split so
-// that the device-scope adds never carry, as flush_limbs does).
-__device__ __forceinline__ void small_flush(const u64* __restrict__ acc, int N, u64* __restrict__ g) {
+// Adds this workgroup's LDS limbs into the device accumulator g (re-split so
+// that the device-scope adds never carry, as flush_limbs does) and clears them.
+__device__ __forceinline__ void small_flush(u64* __restrict__ acc, int N, u64* __restrict__ g) {
     for (int c = threadIdx.x; c < N; c += blockDim.x) {
         const u128 v = limbs_to_u128(acc[c], acc[N + c], acc[2 * N + c]);
+        acc[c] = 0;
+        acc[N + c] = 0;
+        acc[2 * N + c] = 0;
         const u64 l0 = (u64)v & kLimbMask, l1 = (u64)(v >> 43) & kLimbMask, l2 = (u64)(v >> 86);
         if (l0) __hip_atomic_fetch_add(g + 3 * c, l0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (l1) __hip_atomic_fetch_add(g + 3 * c + 1, l1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -545,69 +601,86 @@ __device__ __forceinline__ void small_flush(const u64* __restrict__ acc, int N, 
 // Per-workgroup state of k_small_gauss that is not per particle.
 struct GaussCtl {
     int32_t* okflag;  // LDS: the barrier's verdict for the workgroup
-    uint32_t nblocks, gen;
+    int nblocks;
+    uint32_t gen;
     int64_t nb;       // barriers passed: accumulator nb % 3 is filled before barrier nb
-    bool diagwg;
+    bool diagwg, fit;
+    double iN;
 };
 
 // Deposit of every held particle's centre (the caller's positions), the
 // flush into device accumulator nb % 3, the barrier, and the summed charge
-// staged bit-reversed for the solve.  Returns false if the barrier failed.
+// staged bit-reversed for the solve.  An accumulator is kSmallCopies grids:
+// workgroup b adds into grid b % 8 (its own XCD's), so that adds to one word
+// queue eight deep and not 64, and the readers sum the grids.  Returns false if
+// the barrier failed.
 template <int R, int JMAX>
 __device__ __forceinline__ bool small_deposit_and_meet(const SmallRun& a, const SmallLds& L, GaussCtl& C,
                                                        const double (&cen)[JMAX], const bool (&has)[JMAX], int e) {
+    static_assert(kSmallCopies == 8, "eight lanes sum a cell");
     const InstDesc& I = a.I;
     const int N = I.N;
+    const int64_t copy = 3 * (int64_t)N, set = kSmallCopies * copy;
     if (!C.diagwg) {
-        for (int c = threadIdx.x; c < 3 * N; c += blockDim.x) L.acc[c] = 0;
-        __syncthreads();
 #pragma unroll
         for (int j = 0; j < JMAX; ++j)
-            if (has[j]) seg_deposit<R>(L.acc, N, cen[j], (double)N, I.nmask, I.w, I.q, e);
+            if (has[j]) seg_deposit<R>(L.acc, N, cen[j], (double)N, C.iN, I.nmask, I.w, I.q, C.fit, e);
         __syncthreads();
-        small_flush(L.acc, N, a.gacc + 3 * (int64_t)N * (C.nb % 3));
+        small_flush(L.acc, N, a.gacc + set * (C.nb % 3) + copy * (blockIdx.x % kSmallCopies));
     }
     if (!grid_barrier(a.bar, C.nblocks, C.gen, a.spin_limit, C.okflag)) return false;
     // the accumulator read two barriers ago is free again
-    if (blockIdx.x == 0)
-        for (int c = threadIdx.x; c < 3 * N; c += blockDim.x) st_agent(a.gacc + 3 * (int64_t)N * ((C.nb + 2) % 3) + c, 0);
-    const u64* g = a.gacc + 3 * (int64_t)N * (C.nb % 3);
-    for (int c = threadIdx.x; c < N; c += blockDim.x) {
-        const int b = (int)brev((uint32_t)c, I.log2N);
-        L.re[b] = fxp_to(limbs_to_u128(ld_agent(g + 3 * c), ld_agent(g + 3 * c + 1), ld_agent(g + 3 * c + 2)), I.q);
-        L.im[b] = 0.0;
+    for (int b = blockIdx.x; b < kSmallCopies && !C.diagwg; b += a.K)
+        for (int c = threadIdx.x; c < copy; c += blockDim.x)
+            st_agent(a.gacc + set * ((C.nb + 2) % 3) + copy * b + c, 0);
+    const u64* g = a.gacc + set * (C.nb % 3);
+    for (int i = threadIdx.x; i < kSmallCopies * N; i += blockDim.x) {
+        const int c = i / kSmallCopies;
+        const u64* p = g + copy * (i % kSmallCopies) + 3 * c;
+        const u64 l0 = ld_agent(p), l1 = ld_agent(p + 1), l2 = ld_agent(p + 2);
+        const u64 s0 = sum8_u64(l0), s1 = sum8_u64(l1), s2 = sum8_u64(l2);
+        if (i % kSmallCopies == 0) L.re[(int)brev((uint32_t)c, I.log2N)] = fxp_to(limbs_to_u128(s0, s1, s2), I.q);
     }
     __syncthreads();
     ++C.nb;
     return true;
 }
 
-// Diagnostics workgroup: the row of step `row`, which ended before the last
-// barrier, from the velocities stored then (its field still in Eld).
-__device__ __forceinline__ void small_gauss_diag(const SmallRun& a, const SmallLds& L, int64_t row, int32_t nsweeps,
+// Diagnostics workgroup, one wave per 4096-particle chunk c: the canonical sums
+// of v^2 and v/P of a step that ended before the last barrier, from the
+// velocities stored then, into dp.  Tree lane t = l + 64 u folds particles
+// t + 256 i in order.
+__device__ __forceinline__ void small_chunk_sums(const SmallRun& a, const SmallLds& L, int c, int64_t row,
                                                  int32_t step0) {
-    const InstDesc& I = a.I;
-    const int64_t P = I.P;
-    const int64_t nch = (P + kTreeChunk - 1) / kTreeChunk;
-    const int parw = (int)((step0 + row + 1) & 1);
-    const u64* vg = reinterpret_cast<const u64*>(parw ? a.V1 : a.V0);
-    for (int64_t c = 0; c < nch; ++c) {
-        const int64_t n = (P - c * kTreeChunk) < kTreeChunk ? (P - c * kTreeChunk) : kTreeChunk;
-        const u64* vc = vg + c * kTreeChunk;
-        double s2, s1;
-        chunk_sums_v(L.red, n, (double)P, [&](int64_t i) { return __longlong_as_double((long long)ld_agent(vc + i)); },
-                     s2, s1);
-        if (threadIdx.x == 0) {
-            L.dp[2 * c] = s2;
-            L.dp[2 * c + 1] = s1;
+    const int64_t P = a.I.P, left = P - (int64_t)c * kTreeChunk;
+    const int n = (int)(left < kTreeChunk ? left : kTreeChunk);
+    const u64* v = reinterpret_cast<const u64*>(((step0 + row + 1) & 1) ? a.V1 : a.V0) + (int64_t)c * kTreeChunk;
+    const int l = threadIdx.x & 63;
+    const DivP divP(P);
+    double s2[4] = {0.0, 0.0, 0.0, 0.0}, s1[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int m0 = 0; 64 * m0 < n; m0 += 16) {  // element l + 64 m, m = u + 4 i
+        double x[16];
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+            const int i = l + 64 * (m0 + m);
+            x[m] = i < n ? __longlong_as_double((long long)ld_agent(v + i)) : 0.0;
         }
+#pragma unroll
+        for (int m = 0; m < 16; ++m)
+            if (l + 64 * (m0 + m) < n) {
+                s2[m & 3] = s2[m & 3] + x[m] * x[m];
+                s1[m & 3] = s1[m & 3] + divP(x[m]);
+            }
     }
-    __syncthreads();
-    small_diag_row(L, I, nch, a.diag + 4 * row, a.sweeps + row, nsweeps);
-    __syncthreads();
+    double r[2] = {(s2[0] + s2[2]) + (s2[1] + s2[3]), (s1[0] + s1[2]) + (s1[1] + s1[3])};
+    wave_tree<2>(r, [](int, double p, double q) { return p + q; });
+    if (l == 0) {
+        L.dp[2 * c] = r[0];
+        L.dp[2 * c + 1] = r[1];
+    }
 }
 
-template <int R, int SCHEME>
+template <int R, int SCHEME, int E>
 __global__ void __launch_bounds__(kSmallThreads)
 k_small_gauss(SmallRun a) {
     extern __shared__ double sm[];
@@ -619,10 +692,12 @@ k_small_gauss(SmallRun a) {
     const int K = a.K;
     GaussCtl C;
     C.okflag = &okflag;
-    C.nblocks = (uint32_t)K + 1;
+    C.nblocks = K + 1;
     C.gen = 0;
     C.nb = 0;
     C.diagwg = (int)blockIdx.x == K;
+    C.fit = limbs_fit(I.w, I.q);
+    C.iN = 1.0 / (double)N;
     const int e = threadIdx.x & (kSegLanes - 1);
     const int64_t seg = (int64_t)blockIdx.x * kSegs + (threadIdx.x >> 4);
     const int64_t G = (int64_t)K * kSegs;
@@ -654,10 +729,30 @@ k_small_gauss(SmallRun a) {
             L.Eld[j] = Ein[j];
         }
     }
+    for (int c = threadIdx.x; c < 3 * N; c += blockDim.x) L.acc[c] = 0;
     stage_tables(L, a.tw, N);
+    WaveTables<E> W;
+    load_wave_tables<E>(W, L, N);
     bool bad = false, ok = true;
     int64_t pend_row = -1;  // diagnostics workgroup: step whose row is still to be written
     int32_t pend_sweeps = 0;
+    double pend_se = 0.0;
+    const int nch = (int)((P + kTreeChunk - 1) / kTreeChunk);
+    // The field of the staged charge (wave 0); in the diagnostics workgroup
+    // beside it the sums of the pending step (waves 1..nch) and its row.
+    // Returns the convergence test.
+    auto solve = [&](auto test) {
+        const bool pend = C.diagwg && pend_row >= 0;
+        if (threadIdx.x < 64) wave_solve<decltype(test)::value, E>(L, W, N, log2N, I.rtol);
+        else if (pend && (int)threadIdx.x < 64 * (1 + nch))
+            small_chunk_sums(a, L, (int)(threadIdx.x >> 6) - 1, pend_row, S0.step);
+        __syncthreads();
+        if (pend && threadIdx.x == 0)
+            small_diag_row(L, I, pend_se, nch, a.diag + 4 * pend_row, a.sweeps + pend_row, pend_sweeps);
+        pend_row = -1;
+        bad = bad || !isfinite(L.red[0]);
+        return L.red[1] != 0.0;
+    };
 
     for (int64_t s = 0; s < a.nsteps && ok; ++s) {
         const int paro = (int)((S0.step + s + 1) & 1);
@@ -671,16 +766,14 @@ k_small_gauss(SmallRun a) {
                 cen[j] = (Xp[j] + Xp[j]) / 2.0;
             }
             if (!(ok = small_deposit_and_meet<R, JMAX>(a, L, C, cen, has, e))) break;
-            if (C.diagwg && pend_row >= 0) small_gauss_diag(a, L, pend_row, pend_sweeps, S0.step);
-            double emax;
-            small_solve<false>(L, N, log2N, 0.0, emax);
-            bad = bad || !isfinite(emax);
+            solve(std::false_type{});
+            pend_se = L.red[2];
             // u(); v += gather(E, x)*dt
 #pragma unroll
             for (int j = 0; j < JMAX; ++j)
                 if (has[j]) {
                     Xp[j] = jl_mod1f(Xp[j] + (Vp[j] / 2.0) * dt);
-                    Vp[j] = Vp[j] + seg_gather<R>(L.Eld, Xp[j], Nd, nmask, e) * dt;
+                    Vp[j] = Vp[j] + seg_gather<R>(L.Eld, Xp[j], Nd, C.iN, nmask, e) * dt;
                     if (e == 0) {
                         st_agent(Xo + seg + G * j, (u64)__double_as_longlong(Xp[j]));
                         st_agent(Vo + seg + G * j, (u64)__double_as_longlong(Vp[j]));
@@ -698,11 +791,8 @@ k_small_gauss(SmallRun a) {
                 cen[j] = (x + Xp[j]) / 2.0;
             }
             if (!(ok = small_deposit_and_meet<R, JMAX>(a, L, C, cen, has, e))) break;
-            if (C.diagwg && pend_row >= 0) small_gauss_diag(a, L, pend_row, pend_sweeps, S0.step);
             for (int k = 0;; ++k) {
-                double emax;
-                const bool conv = small_solve<true>(L, N, log2N, I.rtol, emax);
-                bad = bad || !isfinite(emax);
+                const bool conv = solve(std::true_type{});
                 const bool done = conv || k == I.max_sweeps - 1;
                 // v_{k+1} = V + gather(E_k, c_k)*dt; unless the loop ends here
                 // the next centre c_{k+1} = (x_{k+1} + X)/2
@@ -710,7 +800,7 @@ k_small_gauss(SmallRun a) {
                 for (int j = 0; j < JMAX; ++j)
                     if (has[j]) {
                         const double x = Xp[j] + ((vk[j] + Vp[j]) / 2.0) * dt;
-                        const double vn = Vp[j] + seg_gather<R>(L.Eld, (x + Xp[j]) / 2.0, Nd, nmask, e) * dt;
+                        const double vn = Vp[j] + seg_gather<R>(L.Eld, (x + Xp[j]) / 2.0, Nd, C.iN, nmask, e) * dt;
                         if (done) {
                             Xp[j] = jl_mod1f(x);
                             Vp[j] = vn;
@@ -727,6 +817,7 @@ k_small_gauss(SmallRun a) {
                 if (done) {
                     pend_row = s;
                     pend_sweeps = k + 1;
+                    pend_se = L.red[2];
                     break;
                 }
                 if (!(ok = small_deposit_and_meet<R, JMAX>(a, L, C, cen, has, e))) break;
@@ -734,7 +825,12 @@ k_small_gauss(SmallRun a) {
         }
     }
     if (ok) ok = grid_barrier(a.bar, C.nblocks, C.gen, a.spin_limit, C.okflag);
-    if (ok && C.diagwg && pend_row >= 0) small_gauss_diag(a, L, pend_row, pend_sweeps, S0.step);
+    if (ok && C.diagwg && pend_row >= 0) {
+        if ((int)threadIdx.x < 64 * nch) small_chunk_sums(a, L, (int)(threadIdx.x >> 6), pend_row, S0.step);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            small_diag_row(L, I, pend_se, nch, a.diag + 4 * pend_row, a.sweeps + pend_row, pend_sweeps);
+    }
     if (blockIdx.x == 0 && ok) {
         double* Eo = S0.e_cur ? a.E1 : a.E0;
         for (int j = threadIdx.x; j < N; j += blockDim.x) Eo[j] = L.Eld[j];
@@ -773,36 +869,35 @@ int small_workgroups_ok(const InstDesc& I, int64_t K) {
     return K >= 1 && K <= kSmallMaxGroups && (I.P + K * kSegs - 1) / (K * kSegs) <= kSmallMaxSlots;
 }
 
+// the kernel of a shape, scheme and solve width
+template <int E>
+static const void* small_kernel(int R, int scheme) {
+    if (R == 0) return reinterpret_cast<const void*>(k_small_ngp<E>);
+    if (R == 6)
+        return scheme ? reinterpret_cast<const void*>(k_small_gauss<6, 1, E>)
+                      : reinterpret_cast<const void*>(k_small_gauss<6, 0, E>);
+    return scheme ? reinterpret_cast<const void*>(k_small_gauss<7, 1, E>)
+                  : reinterpret_cast<const void*>(k_small_gauss<7, 0, E>);
+}
+
 hipError_t launch_small_run(const SmallRun& a, int scheme, hipStream_t s) {
-    const int lds = small_lds_bytes(a.I.N, a.I.R == 0);
+    const unsigned lds = (unsigned)small_lds_bytes(a.I.N);
     SmallRun arg = a;
     void* args[] = {&arg};
-    if (a.I.R == 0) {
-        k_small_ngp<kSmallNgpSlots><<<1, kSmallThreads, lds, s>>>(a);
-        return hipGetLastError();
-    }
-    const void* f;
-    if (a.I.R == 6) f = scheme ? reinterpret_cast<const void*>(k_small_gauss<6, 1>)
-                               : reinterpret_cast<const void*>(k_small_gauss<6, 0>);
-    else f = scheme ? reinterpret_cast<const void*>(k_small_gauss<7, 1>)
-                    : reinterpret_cast<const void*>(k_small_gauss<7, 0>);
-    return hipLaunchCooperativeKernel(f, dim3((unsigned)a.K + 1), dim3(kSmallThreads), args, (unsigned)lds, s);
+    const void* f = a.I.N <= 64 ? small_kernel<1>(a.I.R, scheme)
+                                : a.I.N <= 128 ? small_kernel<2>(a.I.R, scheme) : small_kernel<4>(a.I.R, scheme);
+    if (a.I.R == 0) return hipLaunchKernel(f, dim3(1), dim3(kSmallThreads), args, lds, s);
+    return hipLaunchCooperativeKernel(f, dim3((unsigned)a.K + 1), dim3(kSmallThreads), args, lds, s);
 }
 
 int configure_kernels_small() {
-    const int bytes = small_lds_bytes(kSmallMaxN, true);
+    const int bytes = small_lds_bytes(kSmallMaxN);
     hipError_t e = hipSuccess;
     auto chk = [&](hipError_t r) { if (r != hipSuccess) e = r; };
-    chk(hipFuncSetAttribute(reinterpret_cast<const void*>(k_small_ngp<kSmallNgpSlots>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    chk(hipFuncSetAttribute(reinterpret_cast<const void*>(k_small_gauss<6, 0>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    chk(hipFuncSetAttribute(reinterpret_cast<const void*>(k_small_gauss<6, 1>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    chk(hipFuncSetAttribute(reinterpret_cast<const void*>(k_small_gauss<7, 0>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
-    chk(hipFuncSetAttribute(reinterpret_cast<const void*>(k_small_gauss<7, 1>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+    for (int R : {0, 6, 7})
+        for (int scheme = 0; scheme < 2; ++scheme)
+            for (const void* f : {small_kernel<1>(R, scheme), small_kernel<2>(R, scheme), small_kernel<4>(R, scheme)})
+                chk(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
     (void)hipGetLastError();
     return e == hipSuccess ? 0 : -1;
 }

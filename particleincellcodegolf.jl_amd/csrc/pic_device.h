@@ -173,7 +173,7 @@ __device__ __forceinline__ double ol_erf(double x) {
 // mod(x, 1) on Float64 (src/NGPFourier.jl:2, src/GaussianFixedPointQuiet.jl:10):
 // r = rem(x, 1); r == 0 -> +0; r < 0 -> r + 1 (rounded); else r.
 __device__ __forceinline__ double jl_mod1f(double x) {
-    double r = fmod(x, 1.0);
+    double r = x - trunc(x);  // fmod(x, 1.0): the fractional part is exact (NaN for infinities, as there)
     if (r == 0.0) return 0.0;
     if (r < 0.0) return r + 1.0;
     return r;

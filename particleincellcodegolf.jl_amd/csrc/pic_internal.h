@@ -154,6 +154,10 @@ constexpr int kSmallMaxN = 256;       // the solve runs in one wave, 4 grid cell
 constexpr int kSmallNgpSlots = 16;    // NGP: particles per thread of the one 512-thread workgroup (P <= 8192)
 constexpr int kSmallMaxSlots = 4;     // Gaussian: particles per 16-lane segment
 constexpr int kSmallMaxGroups = 128;  // Gaussian: particle workgroups (32 segments each; P <= 16384)
+constexpr int kSmallCopies = 8;       // Gaussian: grids of a device charge accumulator
+constexpr int kSmallBarWords = 256;   // Gaussian: the barrier's words, one per workgroup
+constexpr int kSmallAbort = 255;      // ... and the one a workgroup that gave up sets
+static_assert(kSmallMaxGroups + 1 <= kSmallAbort, "one word per workgroup");
 struct SmallRun {
     InstDesc I;
     InstState* st;
@@ -162,8 +166,8 @@ struct SmallRun {
     double* diag;                // nsteps x 4
     int32_t* sweeps;             // nsteps
     int64_t nsteps;
-    unsigned long long* gacc;    // Gaussian: three device charge accumulators of 3N limbs
-    uint32_t* bar;               // Gaussian: barrier counter, generation, failure flag
+    unsigned long long* gacc;    // Gaussian: three device charge accumulators of kSmallCopies x 3N limbs
+    uint32_t* bar;               // Gaussian: kSmallBarWords words of the grid barrier
     int32_t K;                   // Gaussian: particle workgroups (one more computes diagnostics)
     uint32_t spin_limit;         // Gaussian: polls before a barrier wait gives up
 };
