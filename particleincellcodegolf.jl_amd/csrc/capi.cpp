@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/pic.h"
+#include "hostcopy.h"
 #include "pic_internal.h"
 #include "trace.h"
 
@@ -31,6 +32,7 @@ struct DevBuf {
 }  // namespace
 
 struct pic_ctx {
+    bool staging = false;  // holds the device's staging buffers (hostcopy.h)
     int device = 0;
     hipStream_t stream = nullptr;
     std::vector<pic_config> cfg;
@@ -483,6 +485,8 @@ int pic_create_batch(pic_ctx** out, const pic_config* cfgs, int32_t n) {
         if ((rc = dalloc(c, &c->small_gacc, 9 * kSmallCopies * (size_t)c->hinst[0].N))) return fail(rc);
         if ((rc = dalloc(c, &c->small_bar, kSmallBarWords))) return fail(rc);
     }
+    hostcopy_retain(c->device);
+    c->staging = true;
     *out = c;
     return PIC_OK;
 }
@@ -506,6 +510,7 @@ int pic_destroy(pic_ctx* c) {
     if (c->rb.diag) (void)hipFree(c->rb.diag);
     if (c->rb.sweeps) (void)hipFree(c->rb.sweeps);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->staging) hostcopy_release(c->device);
     delete c;
     return PIC_OK;
 }
@@ -589,29 +594,19 @@ int pic_download(pic_ctx* c, int32_t inst, double* x, double* v, double* E) {
     const InstDesc& d = c->hinst[inst];
     const int par = (int)(c->steps_done & 1);
     const size_t P = (size_t)d.P;
+    // the stream's work is done before the copies, which run on streams of
+    // their own
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    CopyOut list[3] = {};
     if (c->precision == PIC_PREC_FP64) {
-        if (x) HIPCHK(c, hipMemcpyAsync(x, c->rb.X[par] + d.poff, P * 8, hipMemcpyDeviceToHost, c->stream));
-        if (v) HIPCHK(c, hipMemcpyAsync(v, c->rb.V[par] + d.poff, P * 8, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-    } else if (x || v) {
-        std::vector<uint32_t> xq(P);
-        std::vector<float> vh(P), vl(P);
-        HIPCHK(c, hipMemcpyAsync(xq.data(), c->rb.Xq[par] + d.poff, P * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipMemcpyAsync(vh.data(), c->rb.Vh[par] + d.poff, P * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipMemcpyAsync(vl.data(), c->rb.Vl[par] + d.poff, P * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (size_t j = 0; j < P; ++j) {
-            if (x) x[j] = (double)xq[j] * 0x1p-32;
-            if (v) v[j] = ((double)vh[j] + (double)vl[j]) * d.inv_vstep;
-        }
+        list[0] = {kCopyF64, x, {c->rb.X[par] + d.poff, nullptr}, P, 1.0, nullptr};
+        list[1] = {kCopyF64, v, {c->rb.V[par] + d.poff, nullptr}, P, 1.0, nullptr};
+    } else {
+        list[0] = {kCopyFix32, x, {c->rb.Xq[par] + d.poff, nullptr}, P, 1.0, nullptr};
+        list[1] = {kCopyPair32, v, {c->rb.Vh[par] + d.poff, c->rb.Vl[par] + d.poff}, P, d.inv_vstep, nullptr};
     }
-    if (E) {
-        std::vector<InstState> st;
-        int rc = read_states(c, st);
-        if (rc) return rc;
-        const double* src = c->rb.E[st[inst].e_cur] + d.goff;
-        HIPCHK(c, hipMemcpy(E, src, sizeof(double) * d.N, hipMemcpyDeviceToHost));
-    }
+    list[2] = {kCopyPickF64, E, {c->rb.E[0] + d.goff, c->rb.E[1] + d.goff}, (size_t)d.N, 1.0, &c->rb.st[inst].e_cur};
+    HIPCHK(c, copy_out(c->device, list, 3));
     return PIC_OK;
 }
 

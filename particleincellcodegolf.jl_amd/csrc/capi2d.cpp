@@ -12,12 +12,14 @@
 #include <vector>
 
 #include "../../include/pic2d.h"
+#include "hostcopy.h"
 #include "pic2d_internal.h"
 #include "trace.h"
 
 using namespace pic;
 
 struct pic2d_ctx {
+    bool staging = false;  // holds the device's staging buffers (hostcopy.h)
     pic2d_config cfg{};
     hipStream_t stream = nullptr;
     Buffers2D b{};
@@ -157,6 +159,7 @@ static void release(pic2d_ctx* c) {
     for (void*& p : c->op)
         if (p) (void)hipFree(p);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->staging) hostcopy_release(c->cfg.device);
     delete c;
 }
 
@@ -312,6 +315,8 @@ extern "C" int pic2d_create(pic2d_ctx** out, const pic2d_config* cfg) {
         hipMemset(b.Ex, 0, G * sizeof(double)) != hipSuccess || hipMemset(b.Ey, 0, G * sizeof(double)) != hipSuccess ||
         hipMemset(b.E32, 0, G * sizeof(float2)) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         return fail(PIC_EHIP);
+    hostcopy_retain(c->cfg.device);
+    c->staging = true;
     *out = c;
     return PIC_OK;
 }
@@ -407,46 +412,30 @@ extern "C" int pic2d_download(pic2d_ctx* c, double* x, double* y, double* vx, do
     }
     HIPCHK(c, hipSetDevice(c->cfg.device));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    const int64_t P = c->cfg.P, G = (int64_t)c->cfg.NX * c->cfg.NY;
+    const size_t P = (size_t)c->cfg.P, G = (size_t)c->cfg.NX * c->cfg.NY;
     Buffers2D& b = c->b;
-    if (c->cfg.precision == PIC_PREC_MIXED) {
-        // held particles are grouped by tile; pid gives each one's caller index
-        std::vector<uint32_t> q(P), id(P);
-        std::vector<float> f(P);
-        HIPCHK(c, hipMemcpy(id.data(), b.pid, 4 * P, hipMemcpyDeviceToHost));
-        auto tx = [&](uint32_t* src, double* dst) -> int {
-            HIPCHK(c, hipMemcpy(q.data(), src, 4 * P, hipMemcpyDeviceToHost));
-            for (int64_t p = 0; p < P; ++p) dst[id[p]] = q[p] ? std::ldexp((double)q[p], -32) : 1.0;
-            return PIC_OK;
-        };
-        int rc;
-        if (x && (rc = tx(b.Xq, x))) return rc;
-        if (y && (rc = tx(b.Yq, y))) return rc;
-        float* ss[3] = {b.VXf, b.VYf, b.VZf};
-        float* sl[3] = {b.VXl, b.VYl, b.VZl};
-        double* ds[3] = {vx, vy, vz};
-        std::vector<float> fl(P);
-        for (int k = 0; k < 3; ++k) {
-            if (!ds[k]) continue;
-            HIPCHK(c, hipMemcpy(f.data(), ss[k], 4 * P, hipMemcpyDeviceToHost));
-            HIPCHK(c, hipMemcpy(fl.data(), sl[k], 4 * P, hipMemcpyDeviceToHost));
-            for (int64_t p = 0; p < P; ++p) ds[k][id[p]] = (double)f[p] + (double)fl[p];
-        }
-    } else {
-        // held by tile too: back to the caller's order through pid
-        std::vector<uint32_t> id(P);
-        std::vector<double> f(P);
-        HIPCHK(c, hipMemcpy(id.data(), b.pid, 4 * P, hipMemcpyDeviceToHost));
-        const double* ss[5] = {b.X, b.Y, b.VX, b.VY, b.VZ};
-        double* ds[5] = {x, y, vx, vy, vz};
-        for (int k = 0; k < 5; ++k) {
-            if (!ds[k]) continue;
-            HIPCHK(c, hipMemcpy(f.data(), ss[k], 8 * P, hipMemcpyDeviceToHost));
-            for (int64_t p = 0; p < P; ++p) ds[k][id[p]] = f[p];
+    std::vector<CopyOut> list;
+    if (x || y || vx || vy || vz) {
+        // held particles are grouped by tile: the regroup's other buffers take
+        // them in the caller's order
+        launch2d_unpermute(b, c->stream);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (c->cfg.precision == PIC_PREC_MIXED) {
+            list.push_back({kCopyUnimod32, x, {b.Xq_alt, nullptr}, P, 1.0, nullptr});
+            list.push_back({kCopyUnimod32, y, {b.Yq_alt, nullptr}, P, 1.0, nullptr});
+            list.push_back({kCopyPair32, vx, {b.VXf_alt, b.VXl_alt}, P, 1.0, nullptr});
+            list.push_back({kCopyPair32, vy, {b.VYf_alt, b.VYl_alt}, P, 1.0, nullptr});
+            list.push_back({kCopyPair32, vz, {b.VZf_alt, b.VZl_alt}, P, 1.0, nullptr});
+        } else {
+            const double* src[5] = {b.X_alt, b.Y_alt, b.VX_alt, b.VY_alt, b.VZ_alt};
+            double* dst[5] = {x, y, vx, vy, vz};
+            for (int k = 0; k < 5; ++k) list.push_back({kCopyF64, dst[k], {src[k], nullptr}, P, 1.0, nullptr});
         }
     }
-    if (Ex) HIPCHK(c, hipMemcpy(Ex, b.Ex, 8 * G, hipMemcpyDeviceToHost));
-    if (Ey) HIPCHK(c, hipMemcpy(Ey, b.Ey, 8 * G, hipMemcpyDeviceToHost));
+    list.push_back({kCopyF64, Ex, {b.Ex, nullptr}, G, 1.0, nullptr});
+    list.push_back({kCopyF64, Ey, {b.Ey, nullptr}, G, 1.0, nullptr});
+    HIPCHK(c, copy_out(c->cfg.device, list.data(), (int)list.size()));
     return PIC_OK;
 }
 

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/pic2d3v.h"
+#include "hostcopy.h"
 #include "pic2d3v_internal.h"
 #include "trace.h"
 #include "pic2d3v_lg_internal.h"
@@ -23,6 +24,7 @@
 using namespace pic;
 
 struct pic2d3v_ctx {
+    bool staging = false;  // holds the device's staging buffers (hostcopy.h)
     pic2d3v_config cfg{};
     hipStream_t stream = nullptr;
     Grid23 g{};
@@ -159,6 +161,7 @@ static void release(pic2d3v_ctx* c) {
     for (void*& p : c->op)
         if (p) (void)hipFree(p);
     if (c->stream) (void)hipStreamDestroy(c->stream);
+    if (c->staging) hostcopy_release(c->cfg.device);
     delete c;
 }
 
@@ -566,6 +569,8 @@ extern "C" int pic2d3v_create(pic2d3v_ctx** out, const pic2d3v_config* cfg) {
         L.ky = ky;
     }
     if ((rc = zero_state(c))) return fail(rc);
+    hostcopy_retain(c->cfg.device);
+    c->staging = true;
     *out = c;
     return PIC_OK;
 }
@@ -638,8 +643,10 @@ extern "C" int pic2d3v_download(pic2d3v_ctx* c, int32_t s, double* xyv) {
     if ((rc = scratch(c, 0, sizeof(double) * 5 * (size_t)sp.P, &st))) return rc;
     if (c->mixed) launch23m_pack(c->g, sp, (double*)st, c->stream);
     else launch23_pack(sp, (double*)st, c->stream);
-    HIPCHK(c, hipMemcpyAsync(xyv, st, sizeof(double) * 5 * (size_t)sp.P, hipMemcpyDeviceToHost, c->stream));
-    return finish(c);
+    if ((rc = finish(c))) return rc;
+    const CopyOut all = {kCopyF64, xyv, {st, nullptr}, 5 * (size_t)sp.P, 1.0, nullptr};
+    HIPCHK(c, copy_out(c->cfg.device, &all, 1));
+    return PIC_OK;
 }
 
 extern "C" int pic2d3v_reset(pic2d3v_ctx* c) {
@@ -1094,9 +1101,11 @@ extern "C" int pic2d3v_fields(pic2d3v_ctx* c, double* Exs, double* Eys, double* 
         if (phis) HIPCHK(c, hipMemcpy(phis, c->lg.bins + PIC2D3V_LG_BIN_PHI * blk, n, hipMemcpyDeviceToHost));
         return PIC_OK;
     }
-    if (Exs) HIPCHK(c, hipMemcpy(Exs, c->d.Exs, n, hipMemcpyDeviceToHost));
-    if (Eys) HIPCHK(c, hipMemcpy(Eys, c->d.Eys, n, hipMemcpyDeviceToHost));
-    if (phis) HIPCHK(c, hipMemcpy(phis, c->d.phis, n, hipMemcpyDeviceToHost));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const CopyOut list[3] = {{kCopyF64, Exs, {c->d.Exs, nullptr}, n / 8, 1.0, nullptr},
+                             {kCopyF64, Eys, {c->d.Eys, nullptr}, n / 8, 1.0, nullptr},
+                             {kCopyF64, phis, {c->d.phis, nullptr}, n / 8, 1.0, nullptr}};
+    HIPCHK(c, copy_out(c->cfg.device, list, 3));
     return PIC_OK;
 }
 
@@ -1233,8 +1242,10 @@ extern "C" int pic2d3v_lg_get(pic2d3v_ctx* c, int32_t which, double* z) {
     }
     HIPCHK(c, hipSetDevice(c->cfg.device));
     const size_t G = (size_t)c->cfg.NX * c->cfg.NY;
-    HIPCHK(c, hipMemcpyAsync(z, c->lg.F + which * G, sizeof(double2) * G, hipMemcpyDeviceToHost, c->stream));
-    return finish(c);
+    if (int rc = finish(c)) return rc;
+    const CopyOut all = {kCopyF64, z, {c->lg.F + which * G, nullptr}, 2 * G, 1.0, nullptr};
+    HIPCHK(c, copy_out(c->cfg.device, &all, 1));
+    return PIC_OK;
 }
 
 extern "C" int pic2d3v_lg_set(pic2d3v_ctx* c, int32_t which, const double* z) {

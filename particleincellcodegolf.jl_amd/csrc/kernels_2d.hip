@@ -915,6 +915,22 @@ k2d_diag_final(double* __restrict__ gpart, int64_t ng, double* __restrict__ ppar
     }
 }
 
+// Held particles back to the caller's order (a download): array k's particle p
+// to place pid[p].
+template <typename T, int K>
+struct Arrays2D {
+    const T* src[K];
+    T* dst[K];
+};
+template <typename T, int K>
+__global__ void __launch_bounds__(256) k2d_unpermute(Arrays2D<T, K> a, const uint32_t* __restrict__ pid, int64_t P) {
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t q = pid[p];
+#pragma unroll
+        for (int k = 0; k < K; ++k) a.dst[k][q] = a.src[k][p];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -951,6 +967,21 @@ void launch2d_tile_sort(const Buffers2D& b, hipStream_t s) {
         k2d_tile_scan<<<1, 1024, 0, s>>>(b.T);
         k2d_tile_scatter64<<<nb, 256, lds, s>>>(b.D, b.T, b.X, b.Y, b.VX, b.VY, b.VZ, b.pid, b.X_alt, b.Y_alt,
                                                 b.VX_alt, b.VY_alt, b.VZ_alt, b.pid_alt, b.slot, per);
+    }
+}
+
+void launch2d_unpermute(const Buffers2D& b, hipStream_t s) {
+    const int64_t P = b.D.P;
+    if (b.precision == 1) {
+        auto f = [](float* p) { return reinterpret_cast<uint32_t*>(p); };
+        const Arrays2D<uint32_t, 8> a = {
+            {b.Xq, b.Yq, f(b.VXf), f(b.VYf), f(b.VZf), f(b.VXl), f(b.VYl), f(b.VZl)},
+            {b.Xq_alt, b.Yq_alt, f(b.VXf_alt), f(b.VYf_alt), f(b.VZf_alt), f(b.VXl_alt), f(b.VYl_alt), f(b.VZl_alt)}};
+        k2d_unpermute<uint32_t, 8><<<push_blocks(P), 256, 0, s>>>(a, b.pid, P);
+    } else {
+        const Arrays2D<double, 5> a = {{b.X, b.Y, b.VX, b.VY, b.VZ},
+                                       {b.X_alt, b.Y_alt, b.VX_alt, b.VY_alt, b.VZ_alt}};
+        k2d_unpermute<double, 5><<<push_blocks(P), 256, 0, s>>>(a, b.pid, P);
     }
 }
 
