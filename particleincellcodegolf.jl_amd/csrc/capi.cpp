@@ -252,17 +252,31 @@ const char* pic_last_error(const pic_ctx* ctx) {
     return ctx ? ctx->err.c_str() : g_create_err.c_str();
 }
 
-// Default tiling: every tile of every instance holds at most tileP particles,
-// so the launch is balanced, with enough tiles to cover the chip.  FP64: as
-// many tiles as fit at once (LDS-bound); mixed: two 1024-thread blocks per CU,
-// so the per-tile partials (N u64 each) stay small.
+// Default tiling: every tile of every instance holds at most tileP particles.
+// FP64: as many tiles as fit at once (LDS-bound).  Mixed, one instance: one
+// 1024-thread block per CU below 8192 particles a block at two (a block's fixed
+// work -- its grid staged, cleared and flushed -- is then half the launch: 83.6
+// against 93.8 us a step at N = 1024, 3e5 particles; 158.8 against 163.1 at
+// N = 4096, 3e6), two beyond (353 against 365 us at 2^24).  Batches: 16 tiles of
+// 512 threads per CU, so that the ends of uneven instances and sweeps that only
+// some instances still need spread out, down to 1536 particles a tile (192
+// instances, 9.2e6 particles: 310 us a step with 2304-particle tiles, 387 with
+// 17984; 40 instances, 1.6e6 particles: 148 with 1664, 155 with 832).
 static void default_tiling(const pic_ctx* c, int64_t* tileP, int* block) {
     const int lds_push = c->scheme == PIC_SCHEME_SIMPSON
                              ? (c->precision == 0 ? simpson_push_lds_bytes(c->maxN) : simpson32_push_lds_bytes(c->maxN))
                              : push_lds_bytes(c->maxN, c->precision);
     const int wg_per_cu = std::max(1, std::min(4, (160 * 1024) / std::max(lds_push, 1)));
-    const int64_t target = (int64_t)c->numCU * (c->precision == 0 ? wg_per_cu : 2);
-    *tileP = (c->Ptot + target - 1) / target;
+    auto per_tile = [&](int64_t tiles_per_cu) {
+        const int64_t target = (int64_t)c->numCU * tiles_per_cu;
+        return (c->Ptot + target - 1) / target;
+    };
+    if (c->ninst > 1) {
+        *tileP = std::max(per_tile(16), std::min<int64_t>(1536, per_tile(2)));
+        *block = 512;
+        return;
+    }
+    *tileP = c->precision == 0 ? per_tile(wg_per_cu) : per_tile(per_tile(2) < 8192 ? 1 : 2);
     *block = (c->precision == 0 && wg_per_cu >= 2) ? 512 : 1024;
 }
 
