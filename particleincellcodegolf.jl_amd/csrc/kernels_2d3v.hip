@@ -46,7 +46,7 @@ k23_push(Grid23 g, Species23 s, const double2* __restrict__ E, u64* __restrict__
     constexpr int n = ShapeCount<SH>::value;
     constexpr int LO = ShapeExtent<SH>::lo, HI = ShapeExtent<SH>::hi;
     __shared__ double2 Ew[kTile23Cells];
-    __shared__ u64 Rw[3 * kTile23Cells];
+    __shared__ u64 Rw[2 * kTile23Cells];  // the charge: lo and hi words (split50)
     __shared__ int red[4][4];
     __shared__ int win[5];
     const int t = threadIdx.x;
@@ -117,11 +117,12 @@ k23_push(Grid23 g, Species23 s, const double2* __restrict__ E, u64* __restrict__
             Ew[e] = E[((ox + rx) & (NX - 1)) + (int64_t)NX * ((oy + ry) & (NY - 1))];
             Rw[e] = 0;
             Rw[kTile23Cells + e] = 0;
-            Rw[2 * kTile23Cells + e] = 0;
         }
     }
     __syncthreads();
     int fb = 0;  // particles that read or added through global memory
+    const double qws = ldexp(s.qw, g.q);
+    const bool fits = split50_fits(s.qw, qws);
 #pragma unroll 1
     for (int k = 0; k < kTile23PPT; ++k) {
         const int64_t p = c0 + t + (int64_t)k * kTile23Threads;
@@ -184,12 +185,14 @@ k23_push(Grid23 g, Species23 s, const double2* __restrict__ E, u64* __restrict__
             in = in && lx[q] < wx && ly[q] < wy;
         }
         fb += in ? 0 : 1;
-        if (in) {
+        if (in && fits && finite23(x, y)) {
 #pragma unroll
             for (int jj = 0; jj < n; ++jj)
 #pragma unroll
-                for (int ii = 0; ii < n; ++ii)
-                    add_limbs_lds(Rw, lx[ii] + wx * ly[jj], fix_round128(wxs[ii] * wys[jj] * s.qw, g.q));
+                for (int ii = 0; ii < n; ++ii) {
+                    u64* w = Rw + lx[ii] + wx * ly[jj];
+                    lds_add50(w, w + kTile23Cells, wxs[ii] * wys[jj] * qws);
+                }
         } else {
 #pragma unroll
             for (int jj = 0; jj < n; ++jj)
@@ -204,10 +207,7 @@ k23_push(Grid23 g, Species23 s, const double2* __restrict__ E, u64* __restrict__
         for (int e = t; e < wx * wy; e += kTile23Threads) {
             const int ry = e / wx, rx = e - ry * wx;
             const int64_t k = ((ox + rx) & (NX - 1)) + (int64_t)NX * ((oy + ry) & (NY - 1));
-            const u64 l0 = Rw[e], l1 = Rw[kTile23Cells + e], l2 = Rw[2 * kTile23Cells + e];
-            if (l0) atomicAdd(racc + k, l0);
-            if (l1) atomicAdd(racc + G + k, l1);
-            if (l2) atomicAdd(racc + 2 * G + k, l2);
+            add_limbs_s(racc, G, k, join50(Rw[e], Rw[kTile23Cells + e]));
         }
     }
 }

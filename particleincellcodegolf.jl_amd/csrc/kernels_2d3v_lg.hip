@@ -45,7 +45,7 @@ namespace pic {
 
 // Window budgets, sized so that four blocks share a CU's 160 KB of LDS: the
 // push stages six doubles per cell (39 KB), the current deposit three grids
-// of three limbs (39 KB).  A chunk of 1024 particles sorted per cell spans
+// of two words (26 KB).  A chunk of 1024 particles sorted per cell spans
 // about 6 x 69 cells with the quadratic B-spline, a regrouped one 13 x 13.
 constexpr int kLGWinCells = 832;
 constexpr int kLGDepCells = 552;
@@ -69,16 +69,18 @@ __device__ __forceinline__ double bits_to_d(u64 b) { return __longlong_as_double
 __device__ __forceinline__ u64 d_to_bits(double d) { return (u64)__double_as_longlong(d); }
 __device__ __forceinline__ double fmax_nn(double a, double b) { return b > a ? b : a; }
 
-// the exact sum of a cell (three 38-bit two's-complement limb counters,
-// modulo 2^114) rounded once
-__device__ __forceinline__ double lg_limbs_v(u64 a0, u64 a1, u64 a2, int q) {
-    u128 v = (u128)a0 + ((u128)a1 << kLimbS) + ((u128)a2 << (2 * kLimbS));
+// the exact sum of a cell (three 38-bit two's-complement limb counters, modulo
+// 2^114) as an integer modulo 2^128, and rounded once
+__device__ __forceinline__ u128 lg_joined(const u64* r, int64_t G, int64_t k) {
+    return (u128)r[k] + ((u128)r[G + k] << kLimbS) + ((u128)r[2 * G + k] << (2 * kLimbS));
+}
+__device__ __forceinline__ double lg_rounded(u128 v, int q) {
     v &= ((u128)1 << (3 * kLimbS)) - 1;
     const i128 s = (v >> (3 * kLimbS - 1)) ? (i128)v - ((i128)1 << (3 * kLimbS)) : (i128)v;
     return i128_to_double(s, q);
 }
 __device__ __forceinline__ double lg_limbs(const u64* r, int64_t G, int64_t k, int q) {
-    return lg_limbs_v(r[k], r[G + k], r[2 * G + k], q);
+    return lg_rounded(lg_joined(r, G, k), q);
 }
 
 // q of a sum bounded by sum_s P_s*(|qw_s|*M_s) (M = 1 for the charge)
@@ -511,7 +513,7 @@ __global__ void __launch_bounds__(kTile23Threads)
 k_lg_deposit(LG23 L, Grid23 g, Species23 s, const double* __restrict__ X, const double* __restrict__ Y) {
     constexpr int n = ShapeCount<SH>::value;
     constexpr int g0 = NG == 1 ? 0 : 1;  // first grid: 0 rho, 1..3 J
-    __shared__ u64 Rw[NG * 3 * kLGDepCells];
+    __shared__ u64 Rw[NG * 2 * kLGDepCells];  // per grid lo and hi words (split50)
     __shared__ int red[4][4];
     __shared__ int win[5];
     const int t = threadIdx.x;
@@ -540,12 +542,11 @@ k_lg_deposit(LG23 L, Grid23 g, Species23 s, const double* __restrict__ X, const 
     const int ox = win[0], oy = win[1], wx = win[2], wy = win[3];
     const bool tile = win[4] != 0;
     if (tile)
-        for (int e = t; e < NG * 3 * kLGDepCells; e += kTile23Threads) Rw[e] = 0;
+        for (int e = t; e < NG * 2 * kLGDepCells; e += kTile23Threads) Rw[e] = 0;
     __syncthreads();
     int q[NG];
 #pragma unroll
     for (int c = 0; c < NG; ++c) q[c] = NG == 1 ? L.qr : lg_frac_bits(L, c);
-    constexpr u64 M = (1ull << kLimbS) - 1;
 #pragma unroll 1
     for (int k = 0; k < kTile23PPT; ++k) {
         const int64_t p = pb + k;
@@ -589,40 +590,49 @@ k_lg_deposit(LG23 L, Grid23 g, Species23 s, const double* __restrict__ X, const 
             ly[qq] = (cy[qq] - oy) & (NY - 1);
             in = in && lx[qq] < wx && ly[qq] < wy;
         }
+        // the window takes every contribution of a particle inside it
+        bool fast = in && finite23(xs[k], ys[k]);
+        double ws[NG];
+#pragma unroll
+        for (int c = 0; c < NG; ++c) {
+            ws[c] = ldexp(w[c], q[c]);
+            fast = fast && split50_fits(w[c], ws[c]);
+        }
+        bool edge = false;  // GHOST: a cell lies outside the interior of the buffered grid
+        if (GHOST)
+#pragma unroll
+            for (int qq = 0; qq < n; ++qq)
+                edge = edge || (unsigned)(ux[qq] - L.b) >= (unsigned)NX || (unsigned)(uy[qq] - L.b) >= (unsigned)NY;
+        if (fast)
+#pragma unroll
+            for (int jj = 0; jj < n; ++jj)
+#pragma unroll
+                for (int ii = 0; ii < n; ++ii) {
+                    const double wxy = wxs[ii] * wys[jj];
+                    u64* r = Rw + lx[ii] + wx * ly[jj];
+#pragma unroll
+                    for (int c = 0; c < NG; ++c)
+                        lds_add50(r + 2 * c * kLGDepCells, r + (2 * c + 1) * kLGDepCells, wxy * ws[c]);
+                }
+        if (fast && !edge) continue;
 #pragma unroll
         for (int jj = 0; jj < n; ++jj)
 #pragma unroll
             for (int ii = 0; ii < n; ++ii) {
                 const double wxy = wxs[ii] * wys[jj];
-                // GHOST: the cell lies outside the interior of the buffered grid
-                const bool ghost = GHOST && ((unsigned)(ux[ii] - L.b) >= (unsigned)NX ||
-                                             (unsigned)(uy[jj] - L.b) >= (unsigned)NY);
+                const bool ghost = edge && ((unsigned)(ux[ii] - L.b) >= (unsigned)NX ||
+                                            (unsigned)(uy[jj] - L.b) >= (unsigned)NY);
+                if (fast && !ghost) continue;
 #pragma unroll
                 for (int c = 0; c < NG; ++c) {
                     const double term = wxy * w[c];
                     if (term == 0.0) continue;
-                    const u128 u = (u128)fix_round128(term, q[c]);
-                    const u64 l[3] = {(u64)u & M, (u64)(u >> kLimbS) & M, (u64)(u >> (2 * kLimbS)) & M};
+                    const i128 v = fix_round128(term, q[c]);
                     if (ghost) {
                         const int64_t Ge = (int64_t)L.NXe * L.NYe;
-                        u64* r = L.eacc + (size_t)(g0 + c) * 3 * Ge;
-                        const int64_t kk = ux[ii] + (int64_t)L.NXe * uy[jj];
-#pragma unroll
-                        for (int b = 0; b < 3; ++b)
-                            if (l[b]) atomicAdd(r + b * Ge + kk, l[b]);
+                        add_limbs_s(L.eacc + (size_t)(g0 + c) * 3 * Ge, Ge, ux[ii] + (int64_t)L.NXe * uy[jj], v);
                     }
-                    if (in) {
-                        const int e = lx[ii] + wx * ly[jj];
-#pragma unroll
-                        for (int b = 0; b < 3; ++b)
-                            if (l[b]) atomicAdd(Rw + (c * 3 + b) * kLGDepCells + e, l[b]);
-                    } else {
-                        u64* r = L.racc + (size_t)(g0 + c) * 3 * G;
-                        const int64_t kk = cx[ii] + (int64_t)NX * cy[jj];
-#pragma unroll
-                        for (int b = 0; b < 3; ++b)
-                            if (l[b]) atomicAdd(r + b * G + kk, l[b]);
-                    }
+                    if (!fast) add_limbs_s(L.racc + (size_t)(g0 + c) * 3 * G, G, cx[ii] + (int64_t)NX * cy[jj], v);
                 }
             }
     }
@@ -633,11 +643,8 @@ k_lg_deposit(LG23 L, Grid23 g, Species23 s, const double* __restrict__ X, const 
             const int64_t k = ((ox + rx) & (NX - 1)) + (int64_t)NX * ((oy + ry) & (NY - 1));
 #pragma unroll
             for (int c = 0; c < NG; ++c)
-#pragma unroll
-                for (int b = 0; b < 3; ++b) {
-                    const u64 v = Rw[(c * 3 + b) * kLGDepCells + e];
-                    if (v) atomicAdd(L.racc + (size_t)(g0 + c) * 3 * G + b * G + k, v);
-                }
+                add_limbs_s(L.racc + (size_t)(g0 + c) * 3 * G, G, k,
+                            join50(Rw[2 * c * kLGDepCells + e], Rw[(2 * c + 1) * kLGDepCells + e]));
         }
 }
 
@@ -943,9 +950,10 @@ void lg_launch_diag_fields(const LG23& L, const Diag23& d, hipStream_t st) {
 // The deposits (k_lg_deposit<.., GHOST>) add every contribution to the
 // periodic limbs racc, as the other fields' deposits do, and a contribution
 // to a ghost cell also to that cell of eacc.  The periodic reduction is then
-// racc itself; an interior buffered cell's counters are its periodic cell's
-// minus those of the cell's ghost images (exact: the counters are sums
-// modulo 2^64), a ghost cell's are eacc's.
+// racc itself; an interior buffered cell's sum is its periodic cell's minus
+// those of the cell's ghost images (exact integers modulo 2^114; limb by limb
+// they do not subtract, since a block's part of racc is carried into limbs
+// once), a ghost cell's is eacc's.
 
 // The value of buffered cell e of component comp (see above)
 __device__ __forceinline__ double si_cell(const LG23& L, int64_t Ge, int comp, int64_t e, const int* q) {
@@ -957,16 +965,13 @@ __device__ __forceinline__ double si_cell(const LG23& L, int64_t Ge, int comp, i
     const int64_t G = (int64_t)NX * NY;
     const int64_t k = (u - b) + (int64_t)NX * (v - b);
     const u64* r = L.racc + (size_t)comp * 3 * G;
-    u64 a0 = r[k], a1 = r[G + k], a2 = r[2 * G + k];
+    u128 sum = lg_joined(r, G, k);
     // the ghost images (u + m NX, v + n NY) of the cell; the cell itself holds 0
     for (int vv = v & (NY - 1); vv < NYe; vv += NY)
         for (int uu = u & (NX - 1); uu < NXe; uu += NX) {
-            const int64_t f = uu + (int64_t)NXe * vv;
-            a0 -= ge[f];
-            a1 -= ge[Ge + f];
-            a2 -= ge[2 * Ge + f];
+            sum -= lg_joined(ge, Ge, uu + (int64_t)NXe * vv);
         }
-    return lg_limbs_v(a0, a1, a2, q[comp]);
+    return lg_rounded(sum, q[comp]);
 }
 
 // The grid rhoJs+ from the limbs into gridP (element i = component i % 4 of

@@ -325,6 +325,37 @@ __host__ __device__ __forceinline__ i128 fix_round128(double a, int q) {
     return (i128)(long long)hi * ((i128)1 << 64) + (i128)(u64)lo;
 }
 
+// fix_round128 for values that a block sums in LDS, as two signed 64-bit words
+// lo + hi 2^50 (|lo| < 2^50, both of the value's sign): t = a 2^q, |t| < 2^100.
+// Splitting in doubles (truncation and fma are exact) takes 10 vector
+// instructions and two LDS adds where the 128-bit integer and its three limbs
+// took some 60 and three: the FP64 deposits of signed charge were bound by
+// those.  A word sums up to 2^12 values without overflow.
+__host__ __device__ __forceinline__ u64 signed_word(double v) {  // an integer-valued double, |v| < 2^51
+    return __builtin_bit_cast(u64, v + 0x1.8p52) - 0x4338000000000000ull;
+}
+__host__ __device__ __forceinline__ void split50(double t, u64& lo, u64& hi) {
+    const double r = __builtin_rint(t);
+    const double h = __builtin_trunc(r * 0x1p-50);
+    hi = signed_word(h);
+    lo = signed_word(__builtin_fma(h, -0x1p50, r));
+}
+__host__ __device__ __forceinline__ i128 join50(u64 lo, u64 hi) {
+    return (i128)(long long)lo + (i128)(long long)hi * ((i128)1 << 50);
+}
+// Whether contributions |c| <= |w| (c = w times weights of at least 2^-212 or
+// 0) may take split50 as c's weight times ws = w 2^q: ws is exact and in range,
+// and neither product is subnormal.
+__host__ __device__ __forceinline__ bool split50_fits(double w, double ws) {
+    return __builtin_fabs(ws) < 0x1p100 && (__builtin_fabs(w) > 0x1p-800 || w == 0.0);
+}
+__device__ __forceinline__ void lds_add50(u64* lo, u64* hi, double t) {
+    u64 l, h;
+    split50(t, l, h);
+    atomicAdd(lo, l);
+    atomicAdd(hi, h);
+}
+
 __device__ __forceinline__ double i128_to_double(i128 v, int q) {
     return v < 0 ? -fxp_to((u128)(-v), q) : fxp_to((u128)v, q);
 }

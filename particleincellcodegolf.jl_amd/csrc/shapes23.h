@@ -217,8 +217,8 @@ __device__ __forceinline__ void deposit23(const Grid23& g, u64* __restrict__ rac
 constexpr int kTile23Threads = 256;
 constexpr int kTile23PPT = 4;
 constexpr int kTile23Chunk = kTile23Threads * kTile23PPT;
-// window cells: 16 B of field + 3 x 8 B of limbs each in the FP64 push
-// (39.4 KB with its bookkeeping: four blocks share a CU's 160 KB)
+// window cells: 16 B of field + 2 x 8 B of charge each in the FP64 push
+// (32 KB: four blocks, which the registers allow, share a CU's 160 KB)
 constexpr int kTile23Cells = 1008;
 constexpr int kTile23Halo = 1;
 
@@ -255,15 +255,8 @@ __device__ __forceinline__ void count_fallback(u64* fallback, int fb) {
     if ((threadIdx.x & 63) == 0 && fb && fallback) atomicAdd(fallback, (u64)fb);
 }
 
-__device__ __forceinline__ void add_limbs_lds(u64* Rw, int idx, i128 v) {
-    const u128 u = (u128)v;
-    constexpr u64 M = (1ull << kLimbS) - 1;
-    const u64 l0 = (u64)u & M;
-    const u64 l1 = (u64)(u >> kLimbS) & M;
-    const u64 l2 = (u64)(u >> (2 * kLimbS)) & M;
-    if (l0) atomicAdd(Rw + idx, l0);
-    if (l1) atomicAdd(Rw + kTile23Cells + idx, l1);
-    if (l2) atomicAdd(Rw + 2 * kTile23Cells + idx, l2);
-}
+// whether a position can be placed on the grid (the fast deposits take only
+// those: contributions of others round to 0, fix_round128)
+__device__ __forceinline__ bool finite23(double x, double y) { return x - x == 0.0 && y - y == 0.0; }
 
 }  // namespace pic
