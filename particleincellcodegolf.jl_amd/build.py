@@ -28,10 +28,13 @@ SOURCES = ["kernels_1d.hip", "kernels_mixed.hip", "kernels_mixed_aux.hip", "kern
 # over five alternating runs (instruction order only; the results are the
 # same bit for bit).  The mixed Simpson push ran about 5% slower under it,
 # so it lives in a unit of its own (kernels_mixed_aux.hip) without it.
-# kernels_1d.hip: hoisting the erf constants out of the particle loops spills
+# The FP64 Gaussian units: hoisting the erf constants out of the particle loops spills
 # 103 scalar registers into vector lanes; without the hoisting the FP64
-# midpoint step (N = 4096, 3e6 particles) takes 1.00 in place of 1.03 ms.
+# midpoint step (N = 4096, 3e6 particles) takes 1.00 in place of 1.03 ms, and
+# the 1D EM push needs 125 vector registers in place of 197.
 EXTRA_FLAGS = {"kernels_1d.hip": ["-mllvm", "-disable-machine-licm"],
+               "kernels_1d2v.hip": ["-mllvm", "-disable-machine-licm"],
+               "kernels_em1d.hip": ["-mllvm", "-disable-machine-licm"],
                "kernels_small.hip": ["-mllvm", "-disable-machine-licm"],
                "kernels_mixed.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
 

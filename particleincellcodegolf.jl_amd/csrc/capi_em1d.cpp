@@ -25,6 +25,8 @@ struct picem1d_ctx {
     std::vector<void*> allocs;
     double* tw = nullptr;
     bool uploaded = false;
+    bool small = false;   // steps by the small chain of kernels
+    bool begun = false;   // its saves of the first step after an upload are made
     int64_t step = 0;
     hipGraphExec_t graph[2] = {nullptr, nullptr};  // without / with the moment fields
     void* op[12] = {};
@@ -183,9 +185,14 @@ extern "C" int picem1d_create(picem1d_ctx** out, const picem1d_config* cfg) {
                         &s.Cy, &s.Cz, &s.ex, &s.ey, &s.ez, &s.by, &s.bz};
     for (double** p : grids)
         if ((rc = dalloc(c, p, N))) return fail(rc);
-    if ((rc = dalloc(c, &s.racc, 30 * (size_t)N)) || (rc = dalloc(c, &s.umax, 8)) ||
+    if ((rc = dalloc(c, &s.racc, 30 * (size_t)N)) || (rc = dalloc(c, &s.umax, 16)) ||
+        (rc = dalloc(c, &s.ticket, 1)) ||
         (rc = dalloc(c, &s.ctl, kEMMaxSweeps + 1)) || (rc = dalloc(c, &s.t, 2)))
         return fail(rc);
+    // the short chain of kernels where none of them has work for the chip
+    c->small = cfg->scheme == PICEM1D_FIXED_POINT && N <= kEMSmallN && P <= kEMSmallP &&
+               cfg->max_sweeps <= kEMSmallSweeps;
+    if (c->small && !cfg->sort && (rc = dalloc(c, &s.tmp, 4 * (size_t)P))) return fail(rc);
     if (cfg->sort) {
         const size_t B = (size_t)s.nb;
         if ((rc = dalloc(c, &s.count, B)) || (rc = dalloc(c, &s.cursor, B)) || (rc = dalloc(c, &s.start, B + 1)) ||
@@ -200,7 +207,8 @@ extern "C" int picem1d_create(picem1d_ctx** out, const picem1d_config* cfg) {
         return fail(PIC_EHIP);
     s.tw = reinterpret_cast<const double2*>(c->tw);
     if (hipMemset(s.racc, 0, sizeof(unsigned long long) * 30 * (size_t)N) != hipSuccess ||
-        hipMemset(s.umax, 0, sizeof(unsigned long long) * 8) != hipSuccess ||
+        hipMemset(s.umax, 0, sizeof(unsigned long long) * 16) != hipSuccess ||
+        hipMemset(s.ticket, 0, sizeof(uint32_t)) != hipSuccess ||
         hipDeviceSynchronize() != hipSuccess)
         return fail(PIC_EHIP);
     *out = c;
@@ -257,7 +265,8 @@ extern "C" int picem1d_upload(picem1d_ctx* c, const double* x, const double* v, 
     const int64_t t[2] = {0, 0};
     HIPCHK(c, hipMemcpy(s.ctl, ctl, sizeof ctl, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(s.t, t, sizeof t, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemset(s.umax, 0, sizeof(unsigned long long) * 8));
+    HIPCHK(c, hipMemset(s.umax, 0, sizeof(unsigned long long) * 16));
+    c->begun = false;
     if (int rc = finish(c)) return rc;
     c->step = 0;
     c->uploaded = true;
@@ -300,6 +309,8 @@ static int capture(picem1d_ctx* c, bool moments, hipGraphExec_t* out) {
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     if (c->cfg.scheme == PICEM1D_EXPLICIT) {
         emx_launch_step(c->s, c->cfg.sort != 0, moments, c->stream);
+    } else if (c->small) {
+        em_launch_small_step(c->s, c->cfg.sort != 0, moments, c->stream);
     } else {
         for (int sw = 0; sw < c->s.max_sweeps; ++sw) em_launch_sweep(c->s, sw, c->stream);
         em_launch_end(c->s, c->cfg.sort != 0, moments, c->stream);
@@ -343,6 +354,10 @@ extern "C" int picem1d_run(picem1d_ctx* c, int64_t nsteps, double* fields, int32
     if (!g && (rc = capture(c, moments, &g))) return rc;
     const int64_t base = c->step;
     HIPCHK(c, hipMemcpyAsync(s.t + 1, &base, sizeof base, hipMemcpyHostToDevice, c->stream));
+    if (c->small && !c->begun) {
+        em_launch_small_begin(s, c->stream);
+        c->begun = true;
+    }
     for (int64_t k = 0; k < nsteps; ++k) HIPCHK(c, hipGraphLaunch(g, c->stream));
     if ((rc = finish(c))) return rc;
     c->step += nsteps;

@@ -15,12 +15,15 @@
 // sort keys), a one-block Gauss and Faraday solve, the sort (X stays
 // unsorted), the split-kick push, the current at (X + x)/2, a one-block Ampere
 // solve, the moments and the step's fields.
+#include <algorithm>
 #include <climits>
 
 #include "fft_lines.h"
 #include "pic_device.h"
 #include "picem1d_internal.h"
 #include "solve1d.h"
+#include "stencil1d.h"
+#include "wave_fft.h"
 
 #pragma clang fp contract(off)
 
@@ -39,18 +42,45 @@ __device__ __forceinline__ int64_t em_irn(double c, int N) {
 }
 
 // s(c) (:9-10): cells mod1(i, N) (0-based) and ff(i, c) for i = irn-6 .. irn+6.
-// Adjacent cells share an edge: ((i+1) - 0.5) equals (i + 0.5) exactly.
+// Adjacent cells share an edge: ((i+1) - 0.5) equals (i + 0.5) exactly.  The
+// centre's cell wraps and c does not, so only a c within half a cell of its
+// wrapped cell has its edges in gauss_edges' intervals; any other is at least
+// N - 1/2 cells away, beyond 6 from every edge for N >= 16: all edges are
+// +-1/2 and the weights 0.
 __device__ __forceinline__ void em_stencil(double c, int N, double Nd, int32_t* cell, double* ff) {
     const int64_t i0 = em_irn(c, N);
-    double lo = ol_erf((((double)(i0 - 6) - 0.5) / Nd - c) * Nd) / 2.0;
+    const double cN = c * Nd, r = rint(cN);
 #pragma unroll
-    for (int k = 0; k < 13; ++k) {
-        const int64_t i = i0 - 6 + k;
-        const double hi = ol_erf((((double)i + 0.5) / Nd - c) * Nd) / 2.0;
-        ff[k] = hi - lo;
-        lo = hi;
-        cell[k] = (int32_t)((i - 1) & (int64_t)(N - 1));
+    for (int k = 0; k < 13; ++k) cell[k] = (int32_t)((i0 - 6 + k - 1) & (int64_t)(N - 1));
+    if (edges_fit(cN) && (double)i0 == r) {
+        double f[14];
+        gauss_edges<6>(c, r, Nd, 1.0 / Nd, f);
+#pragma unroll
+        for (int k = 0; k < 13; ++k) ff[k] = f[k + 1] - f[k];
+    } else if (edges_fit(cN) && N >= 16) {
+#pragma unroll
+        for (int k = 0; k < 13; ++k) ff[k] = 0.0;
+    } else {
+        double lo = ol_erf((((double)(i0 - 6) - 0.5) / Nd - c) * Nd) / 2.0;
+#pragma unroll
+        for (int k = 0; k < 13; ++k) {
+            const double hi = ol_erf((((double)(i0 - 6 + k) + 0.5) / Nd - c) * Nd) / 2.0;
+            ff[k] = hi - lo;
+            lo = hi;
+        }
     }
+}
+
+// The same with one lane of a row of 16 per cell: lane e's weight and cell
+// (lanes 13..15 have none: a weight of no use).
+__device__ __forceinline__ double em_lane_weight(double c, int N, double Nd, double iN, int e, int32_t& cell) {
+    const int64_t i0 = em_irn(c, N);
+    const double cN = c * Nd, r = rint(cN);
+    cell = (int32_t)((i0 - 6 + e - 1) & (int64_t)(N - 1));
+    double f = 0.5;
+    if (edges_fit(cN) && (double)i0 == r) f = gauss_edge<6>(c, r, e, Nd, iN);
+    else if (!(edges_fit(cN) && N >= 16)) f = ol_erf((((double)(i0 - 6 + e) - 0.5) / Nd - c) * Nd) / 2.0;
+    return dpp_f64<0x101>(f, f) - f;  // the next lane's edge
 }
 
 // P*|w|*M*2^q < 2^111
@@ -766,6 +796,494 @@ __global__ void __launch_bounds__(256) k_em_finish(EM1D s) {
 }
 
 // ---------------------------------------------------------------------------
+// The fixed point at the scripts' sizes (P <= kEMSmallP, N <= kEMSmallN): two
+// launches a sweep and two at the step's end, where the general chain has four
+// and three.  At 1024 particles none of these kernels has work for the chip:
+// a step is their latency, and that was a particle's 14 erf in one thread (25
+// us a deposit), one block's transforms through LDS with its twiddles from
+// memory (16 us a solve) and a bitonic sort's 55 barriers (24 us).  Here 16
+// lanes share a particle (one edge each), a wave transforms a line in its
+// registers (wave_fft.h), the particles' ranks are counted, and the last block
+// of a deposit to arrive goes on with what follows it.
+//   k_ems_sweep  the deposits of a sweep; the last block the field updates and
+//                the test (em_wave_solve)
+//   k_ems_push   x of the sweep, the velocities, and the next sweep's midpoints
+//                and current maxima
+//   k_ems_rank   x = mod(x, 1), every particle's rank, the sorted particles
+//                into tmp, the moment maxima
+//   k_ems_end    the particles back, the moments, the next step's saves and
+//                first midpoints; the last block the step's output
+// umax: [0..7] max |uy|, |uz| of sweep k at 2k, 2k + 1 (k < 4); [8..10] the
+// moment maxima.
+// ---------------------------------------------------------------------------
+constexpr int kEMSegs = kEMSmallThreads / 16;  // particles of a block at a time
+
+__device__ __forceinline__ u64 em_ld(const u64* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Whether this block is the last of the launch to arrive (all its threads call;
+// everything the others wrote before is visible then).  Clears the ticket.
+__device__ __forceinline__ bool em_last_block(uint32_t* ticket, int32_t* flag) {
+    wait_memory();  // every wave's adds have been made before thread 0 announces them
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const uint32_t n = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        *flag = n == gridDim.x - 1 ? 1 : 0;
+        if (*flag) {
+            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
+    }
+    __syncthreads();
+    return *flag != 0;
+}
+
+// The exact grids of a block in LDS: grid g's lo and hi words (split50) at
+// 2 g N and (2 g + 1) N.  A contribution of at most M |w| goes there as u ff ws,
+// ws = w 2^q, where the split holds it (|t| < 2^101, see em_fits), else straight
+// into the device limbs.
+struct EMGrid {
+    double w, ws;
+    int q;
+    bool fits;
+};
+__device__ __forceinline__ EMGrid em_grid(const EM1D& s, double M) {
+    EMGrid g;
+    g.w = s.w;
+    g.q = em_frac_bits(s.P, s.w, M);
+    g.ws = ldexp(s.w, g.q);
+    g.fits = fabs(g.ws) < 0x1p200 && M * fabs(g.ws) < 0x1p101 && (fabs(s.w) > 0x1p-800 || s.w == 0.0);
+    return g;
+}
+__device__ __forceinline__ void em_limbs_add(u64* g, int N, int cell, i128 v) {
+    const u128 u = (u128)v;
+    const u64 l0 = (u64)u & kEMLimbMask, l1 = (u64)(u >> kLimbEM) & kEMLimbMask,
+              l2 = (u64)(u >> (2 * kLimbEM)) & kEMLimbMask;
+    if (l0) atomicAdd(g + cell, l0);
+    if (l1) atomicAdd(g + N + cell, l1);
+    if (l2) atomicAdd(g + 2 * N + cell, l2);
+}
+__device__ __forceinline__ void em_put(u64* lds, u64* dev, int N, int cell, const EMGrid& g, double uff) {
+    const double t = uff * g.ws;
+    if (g.fits && fabs(t) < 0x1p101) lds_add50(lds + cell, lds + N + cell, t);
+    else em_limbs_add(dev, N, cell, fix_round128(uff * g.w, g.q));
+}
+// n grids of the block into the device limbs
+__device__ __forceinline__ void em_flush50(const u64* lds, u64* dev, int N, int n) {
+    for (int i = threadIdx.x; i < n * N; i += blockDim.x) {
+        const int g = i / N, c = i - g * N;
+        em_limbs_add(dev + (size_t)3 * N * g, N, c, join50(lds[2 * g * N + c], lds[(2 * g + 1) * N + c]));
+    }
+}
+// the exact sum of a cell, read past this block's caches, and cleared
+__device__ __forceinline__ double em_take(u64* g, int N, int j, int q) {
+    const double v = em_sum(em_ld(g + j), em_ld(g + N + j), em_ld(g + 2 * N + j), q);
+    g[j] = 0;
+    g[N + j] = 0;
+    g[2 * N + j] = 0;
+    return v;
+}
+
+// em_solve_body for N = 64 E points or fewer, a line to a wave: one block of at
+// least three waves and N threads.  Thread j < N keeps cell j.  Returns the
+// test of the next sweep (thread 0's waves; every thread gets it).
+template <int E>
+__device__ bool em_wave_solve(const EM1D& s, int sweep, double* sm) {
+    const int N = s.N, lN = s.lN, t = threadIdx.x, l = t & 63, wv = t >> 6;
+    double* line = sm;            // 5 lines in, then Ex, Ey', Ez' out
+    double* pr = sm + 5 * N;      // the waves' permutations: re, im each
+    double* out = sm + 11 * N;    // 3 lines
+    double* res = sm + 14 * N;    // the test
+    const double sc = 1.0 / (double)N, dt = s.dt, e2 = s.eps * s.eps;
+    double2 w6[6];
+    load_wave_twiddles(w6, s.tw, N);
+    const bool own = t < N;
+    double Fx = 0, Fy = 0, Fz = 0, Cy = 0, Cz = 0;
+    if (own) {
+        const int j = t;
+        const int q0 = em_frac_bits(s.P, s.w, 1.0), q1 = em_frac_bits(s.P, s.w, bits_d(s.umax[2 * sweep])),
+                  q2 = em_frac_bits(s.P, s.w, bits_d(s.umax[2 * sweep + 1]));
+        const double r = em_take(s.racc, N, j, q0), jy = em_take(s.racc + 3 * N, N, j, q1),
+                     jz = em_take(s.racc + 6 * N, N, j, q2);
+        const double By = s.By[j], Bz = s.Bz[j];
+        Fx = s.Ex[j];  // Fx .= Ex (:14)
+        if (sweep == 0) {  // Fy .= Ey; Fz .*= Ez; Cy .= By; Cz .= Bz (:13)
+            Fy = s.Ey[j];
+            Fz = s.Fz[j] * s.Ez[j];
+            Cy = By;
+            Cz = Bz;
+            s.Fy[j] = Fy;
+            s.Fz[j] = Fz;
+            s.Cy[j] = Cy;
+            s.Cz[j] = Cz;
+        } else {
+            Fy = s.Fy[j];
+            Fz = s.Fz[j];
+            Cy = s.Cy[j];
+            Cz = s.Cz[j];
+        }
+        s.Fx[j] = Fx;
+        line[j] = r;
+        line[N + j] = (Bz + Cz) / 2.0;
+        line[2 * N + j] = jy;
+        line[3 * N + j] = (By + Cy) / 2.0;
+        line[4 * N + j] = jz;
+    }
+    __syncthreads();
+    auto load = [&](const double* a, double (&re)[E], double (&im)[E]) {  // bit-reversed, imaginary zero
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            re[q] = i < N ? a[(int)brev((uint32_t)i, lN)] : 0.0;
+            im[q] = 0.0;
+        }
+    };
+    // spectrum (natural order) -> its inverse transform's real parts, scaled, in o
+    auto back = [&](double (&re)[E], double (&im)[E], double* o) {
+        double* pre = pr + 2 * N * wv;
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            if (i < N) {
+                const int p = (int)brev((uint32_t)i, lN);
+                pre[p] = re[q];
+                pre[N + p] = im[q];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            re[q] = i < N ? pre[i] : 0.0;
+            im[q] = i < N ? pre[N + i] : 0.0;
+        }
+        wave_radix2<E>(re, im, w6, s.tw, N, true);
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            if (i < N) o[i] = re[q] * sc;
+        }
+    };
+    if (wv < 3) {  // Gauss; Ampere y; Ampere z (:20-23)
+        double re[E], im[E];
+        load(line + N * (wv == 0 ? 0 : wv == 1 ? 1 : 3), re, im);
+        wave_radix2<E>(re, im, w6, s.tw, N, false);
+        if (wv == 0) {
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int j = q * 64 + l;
+                double kr, ki;
+                ik_of(N, j, kr, ki);
+                const double tt = 1.0 / ki, a = re[q], b = im[q];
+                re[q] = j == 0 ? -0.0 : b * tt;  // (0,0)/(0,0) is NaN; `*= false` keeps its (x86: negative) sign
+                im[q] = j == 0 ? -0.0 : -(a * tt);
+            }
+        } else {
+            double jr[E], ji[E];
+            load(line + N * (wv == 1 ? 2 : 4), jr, ji);
+            wave_radix2<E>(jr, ji, w6, s.tw, N, false);
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                double kr, ki, a, b;
+                ik_of(N, q * 64 + l, kr, ki);
+                cmul(wv == 1 ? -kr : kr, wv == 1 ? -ki : ki, re[q], im[q], a, b);
+                re[q] = a / e2 - jr[q];
+                im[q] = b / e2 - ji[q];
+            }
+        }
+        back(re, im, out + N * wv);
+    }
+    __syncthreads();
+    if (own) {
+        const int j = t;
+        const double Ex = out[j], Ey = Fy + dt * out[N + j], Ez = Fz + dt * out[2 * N + j];
+        const double ey = (Ey + Fy) / 2.0, ez = (Ez + Fz) / 2.0;
+        s.Ex[j] = Ex;
+        s.Ey[j] = Ey;
+        s.Ez[j] = Ez;
+        s.ex[j] = (Ex + Fx) / 2.0;
+        s.ey[j] = ey;
+        s.ez[j] = ez;
+        line[j] = ez;
+        line[N + j] = ey;
+        line[2 * N + j] = Fx;
+        line[3 * N + j] = Ex;
+    }
+    __syncthreads();
+    if (wv < 2) {  // Faraday y, z (:25-27)
+        double re[E], im[E];
+        load(line + N * wv, re, im);
+        wave_radix2<E>(re, im, w6, s.tw, N, false);
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            double kr, ki, a, b;
+            ik_of(N, q * 64 + l, kr, ki);
+            cmul(wv == 0 ? -kr : kr, wv == 0 ? -ki : ki, re[q], im[q], a, b);
+            re[q] = a;
+            im[q] = b;
+        }
+        back(re, im, out + N * wv);
+    } else if (wv == 2) {  // isapprox(Fx, Ex): the test at the top of the next sweep (:14)
+        double f[E], e[E], me, se;
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            f[q] = i < N ? line[2 * N + i] : 0.0;
+            e[q] = i < N ? line[3 * N + i] : 0.0;
+        }
+        const bool conv = wave_isapprox<E>(f, e, N, s.rtol, me, se);
+        if (l == 0) res[0] = conv ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    if (own) {
+        const int j = t;
+        const double By = Cy - dt * out[j], Bz = Cz - dt * out[N + j];
+        s.By[j] = By;
+        s.Bz[j] = Bz;
+        s.by[j] = (By + Cy) / 2.0;
+        s.bz[j] = (Bz + Cz) / 2.0;
+    }
+    return res[0] != 0.0;
+}
+__host__ __device__ constexpr int em_wave_lds(int N) { return 14 * N + 2; }  // doubles
+
+// d((X+x)/2), d((X+x)/2, (V2+v2)/2), d((X+x)/2, (V3+v3)/2) (:20, :22, :23),
+// then in the last block the field updates and the test
+template <int E>
+__global__ void __launch_bounds__(kEMSmallThreads) k_ems_sweep(EM1D s, int sweep) {
+    extern __shared__ double smd[];
+    __shared__ int32_t last;
+    if (s.ctl[sweep] == 0) return;
+    u64* ldsu = reinterpret_cast<u64*>(smd);
+    const int N = s.N;
+    for (int i = threadIdx.x; i < 6 * N; i += blockDim.x) ldsu[i] = 0;
+    __syncthreads();
+    const double Nd = (double)N, iN = 1.0 / Nd;
+    const EMGrid g0 = em_grid(s, 1.0), g1 = em_grid(s, bits_d(s.umax[2 * sweep])),
+                 g2 = em_grid(s, bits_d(s.umax[2 * sweep + 1]));
+    const int e = threadIdx.x & 15;
+    for (int64_t p = (int64_t)blockIdx.x * kEMSegs + (threadIdx.x >> 4); p < s.P; p += (int64_t)gridDim.x * kEMSegs) {
+        const double c = s.c[p];
+        const double uy = (s.V2[p] + s.v2[p]) / 2.0, uz = (s.V3[p] + s.v3[p]) / 2.0;
+        int32_t cell;
+        const double ff = em_lane_weight(c, N, Nd, iN, e, cell);
+        if (e < 13 && ff != 0.0) {
+            em_put(ldsu, s.racc, N, cell, g0, ff);
+            em_put(ldsu + 2 * N, s.racc + 3 * N, N, cell, g1, uy * ff);
+            em_put(ldsu + 4 * N, s.racc + 6 * N, N, cell, g2, uz * ff);
+        }
+    }
+    __syncthreads();
+    em_flush50(ldsu, s.racc, N, 3);
+    if (!em_last_block(s.ticket, &last)) return;
+    const bool conv = em_wave_solve<E>(s, sweep, smd);
+    if (threadIdx.x == 0) {
+        s.ctl[kEMMaxSweeps] += 1;
+        if (sweep + 1 < s.max_sweeps) s.ctl[sweep + 1] = conv ? 0 : 1;
+        s.umax[2 * sweep] = 0;
+        s.umax[2 * sweep + 1] = 0;
+    }
+}
+
+// The block's maxima of non-negative doubles into dst[0..K), as bits.
+template <int K>
+__device__ __forceinline__ void em_block_max(const double (&v)[K], u64* dst, u64* red) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        double r[1] = {v[k]};
+        wave_tree<1>(r, [](int, double a, double b) { return fmax_num(a, b); });
+        if ((threadIdx.x & 63) == 0) red[k * 16 + (threadIdx.x >> 6)] = d_bits(r[0]);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < K) {
+        u64 m = 0;
+        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = max(m, red[threadIdx.x * 16 + w]);
+        atomicMax(dst + threadIdx.x, m);
+    }
+}
+
+// x = X + ((V1 + v1)/2)*dt of the sweep, v at its midpoint (:28-29), and the
+// next sweep's midpoint and maxima
+__global__ void __launch_bounds__(kEMSmallThreads) k_ems_push(EM1D s, int sweep) {
+    extern __shared__ double fe[];
+    __shared__ u64 red[2 * 16];
+    if (s.ctl[sweep] == 0) return;
+    stage_fields(fe, s);
+    const int N = s.N, e = threadIdx.x & 15;
+    const double Nd = (double)N, iN = 1.0 / Nd, dt = s.dt;
+    double m[2] = {0.0, 0.0};
+    for (int64_t p = (int64_t)blockIdx.x * kEMSegs + (threadIdx.x >> 4); p < s.P; p += (int64_t)gridDim.x * kEMSegs) {
+        const double X = s.X[p], u1 = s.V1[p], u2 = s.V2[p], u3 = s.V3[p], v1o = s.v1[p];
+        const double x = X + (u1 + v1o) / 2.0 * dt;
+        int32_t cell;
+        const double ff = em_lane_weight((X + x) / 2.0, N, Nd, iN, e, cell);
+        // the six sums, folded left over the cells (Bx is the script's zero array)
+        const double t[6] = {fe[cell] * ff,     fe[N + cell] * ff,     fe[2 * N + cell] * ff,
+                             0.0 * ff,          fe[3 * N + cell] * ff, fe[4 * N + cell] * ff};
+        double a[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            double S = dpp_f64<0x150>(t[k], t[k]);
+#define PIC_FOLD(q) S = S + dpp_f64<0x150 + q>(t[k], t[k])
+            PIC_FOLD(1); PIC_FOLD(2); PIC_FOLD(3); PIC_FOLD(4); PIC_FOLD(5); PIC_FOLD(6);
+            PIC_FOLD(7); PIC_FOLD(8); PIC_FOLD(9); PIC_FOLD(10); PIC_FOLD(11); PIC_FOLD(12);
+#undef PIC_FOLD
+            a[k] = S;
+        }
+        const double w1 = u1 + a[0] * dt / 2.0, w2 = u2 + a[1] * dt / 2.0, w3 = u3 + a[2] * dt / 2.0;
+        const double c1 = w2 * a[5] - w3 * a[4], c2 = w3 * a[3] - w1 * a[5], c3 = w1 * a[4] - w2 * a[3];
+        const double v1 = u1 + (a[0] + c1) * dt, v2 = u2 + (a[1] + c2) * dt, v3 = u3 + (a[2] + c3) * dt;
+        const double xn = X + (u1 + v1) / 2.0 * dt;
+        m[0] = fmax_num(m[0], fabs((u2 + v2) / 2.0));
+        m[1] = fmax_num(m[1], fabs((u3 + v3) / 2.0));
+        if (e == 0) {
+            s.x[p] = x;
+            s.v1[p] = v1;
+            s.v2[p] = v2;
+            s.v3[p] = v3;
+            s.c[p] = (X + xn) / 2.0;
+        }
+    }
+    if (sweep + 1 < s.max_sweeps) em_block_max<2>(m, s.umax + 2 * (sweep + 1), red);
+}
+
+// x .= mod.(x, 1); p = sortperm(x); x = x[p]; v = v[p, :] (:41) into tmp: a
+// particle's place is the number of particles before it by (key, index), counted
+// by 16 lanes over all keys in LDS -- the stable sort's order.  SORT false: the
+// wrap alone.  The moment maxima.
+template <bool SORT>
+__global__ void __launch_bounds__(kEMSmallThreads) k_ems_rank(EM1D s) {
+    __shared__ u64 key[SORT ? kEMSmallP : 1];
+    __shared__ u64 red[3 * 16];
+    const int P = (int)s.P, e = threadIdx.x & 15;
+    if (SORT) {
+        for (int i = threadIdx.x; i < P; i += blockDim.x) key[i] = em_order_key(jl_mod1f(s.x[i]));
+        __syncthreads();
+    }
+    double m[3] = {0.0, 0.0, 0.0};
+    for (int p = blockIdx.x * kEMSegs + (threadIdx.x >> 4); p < P; p += (int)gridDim.x * kEMSegs) {
+        int rank = p;
+        if (SORT) {
+            const u64 k = key[p];
+            rank = 0;
+            for (int i = e; i < P; i += 16) {
+                const u64 o = key[i];
+                rank += (o < k || (o == k && i < p)) ? 1 : 0;
+            }
+#pragma unroll
+            for (int h = 8; h > 0; h >>= 1) rank += __shfl_xor(rank, h, 16);
+        }
+        const double v1 = s.v1[p], v2 = s.v2[p], v3 = s.v3[p];
+        m[0] = fmax_num(m[0], fabs(v1));
+        m[1] = fmax_num(m[1], fabs(v2));
+        m[2] = fmax_num(m[2], fabs(v3));
+        if (e < 4) s.tmp[(size_t)e * P + rank] = e == 0 ? jl_mod1f(s.x[p]) : e == 1 ? v1 : e == 2 ? v2 : v3;
+        if (SORT && e == 4) s.perm[rank] = (uint32_t)p;
+    }
+    em_block_max<3>(m, s.umax + kEMMomentMax, red);
+}
+
+// The step's saves X .= x, V .= v (:13), the first midpoint and its maxima
+__device__ __forceinline__ void em_begin_one(const EM1D& s, int64_t p, double x, double v1, double v2, double v3,
+                                             double (&m)[2], bool write) {
+    const double xn = x + (v1 + v1) / 2.0 * s.dt;
+    m[0] = fmax_num(m[0], fabs((v2 + v2) / 2.0));
+    m[1] = fmax_num(m[1], fabs((v3 + v3) / 2.0));
+    if (!write) return;
+    s.X[p] = x;
+    s.V1[p] = v1;
+    s.V2[p] = v2;
+    s.V3[p] = v3;
+    s.c[p] = (x + xn) / 2.0;
+}
+
+// the first step after an upload
+__global__ void __launch_bounds__(kEMSmallThreads) k_ems_begin(EM1D s) {
+    __shared__ u64 red[2 * 16];
+    double m[2] = {0.0, 0.0};
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.P; p += (int64_t)gridDim.x * blockDim.x)
+        em_begin_one(s, p, s.x[p], s.v1[p], s.v2[p], s.v3[p], m, true);
+    em_block_max<2>(m, s.umax, red);
+}
+
+template <bool MOMENTS>
+__global__ void __launch_bounds__(kEMSmallThreads) k_ems_end(EM1D s) {
+    extern __shared__ u64 ldsu[];
+    __shared__ u64 red[2 * 16];
+    __shared__ int32_t last;
+    const int N = s.N, P = (int)s.P, e = threadIdx.x & 15;
+    const double Nd = (double)N, iN = 1.0 / Nd;
+    EMGrid g[7];
+    if (MOMENTS) {
+        for (int i = threadIdx.x; i < 14 * N; i += blockDim.x) ldsu[i] = 0;
+        g[0] = em_grid(s, 1.0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const double M = bits_d(s.umax[kEMMomentMax + k]);
+            g[1 + k] = em_grid(s, M);
+            g[4 + k] = em_grid(s, M * M);
+        }
+        __syncthreads();
+    }
+    double m[2] = {0.0, 0.0};
+    for (int p = blockIdx.x * kEMSegs + (threadIdx.x >> 4); p < P; p += (int)gridDim.x * kEMSegs) {
+        const double x = s.tmp[p], v1 = s.tmp[(size_t)P + p], v2 = s.tmp[2 * (size_t)P + p], v3 = s.tmp[3 * (size_t)P + p];
+        em_begin_one(s, p, x, v1, v2, v3, m, e == 0);
+        if (e == 0) {
+            s.x[p] = x;
+            s.v1[p] = v1;
+            s.v2[p] = v2;
+            s.v3[p] = v3;
+        }
+        if (MOMENTS) {
+            int32_t cell;
+            const double ff = em_lane_weight(x, N, Nd, iN, e, cell);
+            if (e < 13 && ff != 0.0) {
+                const double u[7] = {1.0, v1, v2, v3, v1 * v1, v2 * v2, v3 * v3};
+#pragma unroll
+                for (int k = 0; k < 7; ++k)
+                    em_put(ldsu + 2 * k * N, s.racc + (9 + 3 * k) * N, N, cell, g[k], k == 0 ? ff : u[k] * ff);
+            }
+        }
+    }
+    em_block_max<2>(m, s.umax, red);
+    if (MOMENTS) {
+        __syncthreads();
+        em_flush50(ldsu, s.racc + 9 * N, N, 7);
+    }
+    if (!em_last_block(s.ticket, &last)) return;
+    // the step's output slot (fields[:, t, 1:12]) and the next step's flags
+    const int64_t slot = s.t[0] - s.t[1];
+    const bool keep = slot >= 0 && slot < s.out_cap;
+    double* o = s.out + (keep ? slot : 0) * 12 * N;
+    for (int i = threadIdx.x; i < 12 * N; i += blockDim.x) {
+        const int f = i / N, j = i - f * N;
+        if (f < 5) {
+            const double* src = f == 0 ? s.Ex : f == 1 ? s.Ey : f == 2 ? s.Ez : f == 3 ? s.By : s.Bz;
+            if (keep) o[i] = src[j];
+        } else if (MOMENTS) {
+            int q = g[0].q;
+#pragma unroll
+            for (int k = 1; k < 7; ++k) q = f - 5 == k ? g[k].q : q;
+            const double v = em_take(s.racc + (9 + 3 * (f - 5)) * N, N, j, q);
+            if (keep) o[i] = v;
+        }
+    }
+    if (threadIdx.x == 0) {
+        if (keep) s.sweeps_out[slot] = s.ctl[kEMMaxSweeps];
+        s.t[0] += 1;
+        s.ctl[0] = 1;
+        for (int k = 1; k <= kEMMaxSweeps; ++k) s.ctl[k] = 0;
+        for (int k = 2; k < kEMMomentMax + 3; ++k) s.umax[k] = 0;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // the explicit scheme (src/GaussianEMExplicit.jl:12-30)
 // ---------------------------------------------------------------------------
 // X .= x; d(X) into the exact limbs (:13); x .= mod.(X .+ v[:,1]*dt, 1)
@@ -1124,6 +1642,29 @@ static unsigned em_blocks(int64_t n) {
 }
 
 size_t em_solve_lds_bytes(int N) { return sizeof(double) * (10 * (size_t)(N + (N >> 4)) + kRedDoubles); }
+
+// The small chain: blocks of 64 particles
+static unsigned em_small_blocks(const EM1D& s) { return (unsigned)((s.P + kEMSegs - 1) / kEMSegs); }
+
+void em_launch_small_begin(const EM1D& s, hipStream_t st) {
+    k_ems_begin<<<(unsigned)((s.P + kEMSmallThreads - 1) / kEMSmallThreads), kEMSmallThreads, 0, st>>>(s);
+}
+
+void em_launch_small_step(const EM1D& s, bool sort, bool moments, hipStream_t st) {
+    const unsigned nb = em_small_blocks(s);
+    const size_t N = (size_t)s.N;
+    const size_t lds = sizeof(double) * std::max<size_t>(6 * N, em_wave_lds(s.N));
+    for (int sweep = 0; sweep < s.max_sweeps; ++sweep) {
+        if (s.N <= 64) k_ems_sweep<1><<<nb, kEMSmallThreads, lds, st>>>(s, sweep);
+        else if (s.N <= 128) k_ems_sweep<2><<<nb, kEMSmallThreads, lds, st>>>(s, sweep);
+        else k_ems_sweep<4><<<nb, kEMSmallThreads, lds, st>>>(s, sweep);
+        k_ems_push<<<nb, kEMSmallThreads, sizeof(double) * 5 * N, st>>>(s, sweep);
+    }
+    if (sort) k_ems_rank<true><<<nb, kEMSmallThreads, 0, st>>>(s);
+    else k_ems_rank<false><<<nb, kEMSmallThreads, 0, st>>>(s);
+    if (moments) k_ems_end<true><<<nb, kEMSmallThreads, sizeof(u64) * 14 * N, st>>>(s);
+    else k_ems_end<false><<<nb, kEMSmallThreads, 0, st>>>(s);
+}
 
 void em_launch_sweep(const EM1D& s, int sweep, hipStream_t st) {
     const unsigned nb = em_blocks(s.P);

@@ -21,6 +21,14 @@ constexpr int kEMSmallSort = 4096;  // particles the one-block sort takes (the b
 constexpr int kLimbEM = 38;         // exact sums: three 38-bit two's-complement limbs per cell
 constexpr int kEMMaxSweeps = 8;     // ctl[s] = sweep s active; ctl[kEMMaxSweeps] = sweeps run this step
 
+// the small chain of the fixed point (see kernels_em1d.hip): at most this many
+// cells (a line in a wave), particles (their keys in LDS) and sweeps
+constexpr int kEMSmallN = 256;
+constexpr int kEMSmallP = 4096;
+constexpr int kEMSmallSweeps = 4;
+constexpr int kEMSmallThreads = 1024;
+constexpr int kEMMomentMax = 8;     // its moment maxima in umax
+
 // Device state of one context (all pointers device memory).
 struct EM1D {
     int32_t N, lN, max_sweeps, tile;
@@ -33,7 +41,8 @@ struct EM1D {
     double *Fx, *Fy, *Fz, *Cy, *Cz;
     double *ex, *ey, *ez, *by, *bz;
     unsigned long long* racc;   // 10 grids x 3 limbs x N: rho, Jy, Jz, then the 7 moments
-    unsigned long long* umax;   // [8]: max |uy|, |uz| of the sweep; max |v1|, |v2|, |v3| of the step's end
+    uint32_t* ticket;           // arrivals of the small chain's blocks
+    unsigned long long* umax;   // [16]; the general chain [8]: max |uy|, |uz| of the sweep; max |v1|, |v2|, |v3| of the step's end
     int32_t* ctl;               // [kEMMaxSweeps + 1]: sweep s active, sweeps run this step
     int64_t* t;                 // [2]: steps since upload, step of the run call's first output slot
     double* out;                // out_cap slots of 12 x N
@@ -48,6 +57,9 @@ struct EM1D {
 };
 
 void em_launch_sweep(const EM1D& s, int sweep, hipStream_t st);
+// one step of the small chain, and the saves of the first step after an upload
+void em_launch_small_step(const EM1D& s, bool sort, bool moments, hipStream_t st);
+void em_launch_small_begin(const EM1D& s, hipStream_t st);
 void em_launch_end(const EM1D& s, bool sort, bool moments, hipStream_t st);
 // one step of the explicit scheme
 void emx_launch_step(const EM1D& s, bool sort, bool moments, hipStream_t st);

@@ -11,6 +11,12 @@
 
 namespace pic {
 
+// Waits until the wave's stores and atomics have reached the level they are
+// performed at.  Before one thread of a block announces the block's work to
+// others with an agent-scope release: a block barrier alone does not wait for
+// the other waves' outstanding stores.
+__device__ __forceinline__ void wait_memory() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // x of the lane that DPP control CTRL names, `old` in the 4-lane banks of a
 // row that BANKS leaves out
 template <int CTRL, int BANKS = 0xf>
