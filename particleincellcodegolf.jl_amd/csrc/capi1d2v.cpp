@@ -19,6 +19,7 @@ using namespace pic;
 
 namespace {
 constexpr int64_t kSteps12 = 8;  // steps in the long step graph
+constexpr int64_t kSmallSteps12 = 2 * kSmallTurns12;  // one-launch steps in theirs
 }
 
 struct pic1d2v_ctx {
@@ -29,6 +30,7 @@ struct pic1d2v_ctx {
     double* tw = nullptr;
     bool uploaded[2] = {false, false};
     bool primed = false;     // the accumulator holds the charge of the current positions
+    bool small = false;      // steps of one launch each
     int64_t step = 0;        // steps since the upload
     hipGraphExec_t g_one = nullptr, g_many = nullptr;
     void* op[4] = {};
@@ -195,7 +197,9 @@ int pic1d2v_create(pic1d2v_ctx** out, const pic1d2v_config* cfg) {
     b.precision = cfg->precision;
     b.nchunks = ((int64_t)P + kTreeChunk - 1) / kTreeChunk;
     if (b.precision == PIC_PREC_FP64) {
-        if ((rc = dalloc(c, &b.x, NP)) || (rc = dalloc(c, &b.vx, NP)) || (rc = dalloc(c, &b.vy, NP))) return fail(rc);
+        c->small = b.N <= kSmallN12 && (int64_t)NP <= kSmallP12;
+        const size_t NV = c->small ? 2 * NP : NP;
+        if ((rc = dalloc(c, &b.x, NP)) || (rc = dalloc(c, &b.vx, NV)) || (rc = dalloc(c, &b.vy, NV))) return fail(rc);
     } else {
         // the mixed state; velocities in steps of the 2^-32 position grid
         b.vstep = cfg->dt * 4294967296.0;
@@ -217,11 +221,11 @@ int pic1d2v_create(pic1d2v_ctx** out, const pic1d2v_config* cfg) {
             return fail(PIC_EHIP);
         }
     }
-    if ((rc = dalloc(c, &b.racc, 6 * N))) return fail(rc);
+    if ((rc = dalloc(c, &b.racc, 6 * N * (c->small ? 3 : 1)))) return fail(rc);
     if ((rc = dalloc(c, &b.E, N))) return fail(rc);
     if ((rc = dalloc(c, &b.dpart, 3 * (size_t)b.nchunks))) return fail(rc);
     if ((rc = dalloc(c, &b.st, 1))) return fail(rc);
-    if (hipMemset(b.racc, 0, 48 * N) != hipSuccess || hipMemset(b.E, 0, 8 * N) != hipSuccess ||
+    if (hipMemset(b.racc, 0, 48 * N * (c->small ? 3 : 1)) != hipSuccess || hipMemset(b.E, 0, 8 * N) != hipSuccess ||
         hipMemset(b.st, 0, sizeof(State12)) != hipSuccess) {
         set_err(c, "pic1d2v_create: hipMemset failed");
         return fail(PIC_EHIP);
@@ -270,6 +274,11 @@ int pic1d2v_upload(pic1d2v_ctx* c, int32_t species, const double* x, const doubl
     const size_t P = (size_t)c->cfg.P, off = (size_t)species * P;
     Buffers12& b = c->b;
     if (b.precision == PIC_PREC_FP64) {
+        // step 0 reads the first copy of the velocities: another species' may be in the second
+        if (c->small && (c->step & 1))
+            for (double* v : {b.vx, b.vy})
+                HIPCHK(c, hipMemcpyAsync(v, v + (size_t)c->cfg.nspecies * P, 8 * (size_t)c->cfg.nspecies * P,
+                                         hipMemcpyDeviceToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(b.x + off, x, 8 * P, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(b.vx + off, vx, 8 * P, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(b.vy + off, vy, 8 * P, hipMemcpyHostToDevice, c->stream));
@@ -298,7 +307,7 @@ int pic1d2v_upload(pic1d2v_ctx* c, int32_t species, const double* x, const doubl
     }
     // the run restarts: step 0, no field bins or diagnostics, charge to be deposited
     HIPCHK(c, hipMemsetAsync(c->b.st, 0, sizeof(State12), c->stream));
-    HIPCHK(c, hipMemsetAsync(c->b.racc, 0, 48 * (size_t)c->cfg.N, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->b.racc, 0, 48 * (size_t)c->cfg.N * (c->small ? 3 : 1), c->stream));
     if (c->b.Es) HIPCHK(c, hipMemsetAsync(c->b.Es, 0, 8 * (size_t)c->b.cap_bins * c->cfg.N, c->stream));
     if (c->b.D) HIPCHK(c, hipMemsetAsync(c->b.D, 0, 40 * (size_t)c->b.cap_bins, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -320,8 +329,9 @@ int pic1d2v_download(pic1d2v_ctx* c, int32_t species, double* x, double* vx, dou
     const Buffers12& b = c->b;
     if (b.precision == PIC_PREC_FP64) {
         if (x) HIPCHK(c, hipMemcpyAsync(x, b.x + off, 8 * P, hipMemcpyDeviceToHost, c->stream));
-        if (vx) HIPCHK(c, hipMemcpyAsync(vx, b.vx + off, 8 * P, hipMemcpyDeviceToHost, c->stream));
-        if (vy) HIPCHK(c, hipMemcpyAsync(vy, b.vy + off, 8 * P, hipMemcpyDeviceToHost, c->stream));
+        const size_t voff = off + (c->small && (c->step & 1) ? (size_t)c->cfg.nspecies * P : 0);
+        if (vx) HIPCHK(c, hipMemcpyAsync(vx, b.vx + voff, 8 * P, hipMemcpyDeviceToHost, c->stream));
+        if (vy) HIPCHK(c, hipMemcpyAsync(vy, b.vy + voff, 8 * P, hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         return PIC_OK;
     }
@@ -379,7 +389,9 @@ static void enqueue_step(pic1d2v_ctx* c) {
 static int capture(pic1d2v_ctx* c, int64_t steps, hipGraphExec_t* out) {
     hipGraph_t g = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int64_t i = 0; i < steps; ++i) enqueue_step(c);
+    for (int64_t i = 0; i < steps; ++i)
+        if (c->small) launch12_small(c->b, (int)(i % kSmallTurns12), c->stream);
+        else enqueue_step(c);
     HIPCHK(c, hipStreamEndCapture(c->stream, &g));
     const hipError_t e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
@@ -410,14 +422,26 @@ int pic1d2v_run(pic1d2v_ctx* c, int64_t nsteps, double* D) {
         launch12_deposit(c->b, c->stream);
         c->primed = true;
     }
-    int64_t left = nsteps;
-    if (left >= kSteps12 && !c->g_many && (rc = capture(c, kSteps12, &c->g_many))) return rc;
-    if (!c->g_one && (rc = capture(c, 1, &c->g_one))) return rc;
-    while (left >= kSteps12) {
-        HIPCHK(c, hipGraphLaunch(c->g_many, c->stream));
-        left -= kSteps12;
+    if (c->small) {
+        // the graph's turns are those of a step number that kSmallTurns12 divides
+        auto one = [&](int64_t step) { launch12_small(c->b, (int)(step % kSmallTurns12), c->stream); };
+        const int64_t end = c->step + nsteps;
+        int64_t at = c->step;
+        while (at < end && at % kSmallTurns12) one(at++);
+        if (end - at >= kSmallSteps12 && !c->g_many && (rc = capture(c, kSmallSteps12, &c->g_many))) return rc;
+        for (; end - at >= kSmallSteps12; at += kSmallSteps12) HIPCHK(c, hipGraphLaunch(c->g_many, c->stream));
+        while (at < end) one(at++);
+        if (end % c->b.bin == 0) launch12_small_row(c->b, (int)(end % kSmallTurns12), c->stream);
+    } else {
+        int64_t left = nsteps;
+        if (left >= kSteps12 && !c->g_many && (rc = capture(c, kSteps12, &c->g_many))) return rc;
+        if (!c->g_one && (rc = capture(c, 1, &c->g_one))) return rc;
+        while (left >= kSteps12) {
+            HIPCHK(c, hipGraphLaunch(c->g_many, c->stream));
+            left -= kSteps12;
+        }
+        while (left-- > 0) HIPCHK(c, hipGraphLaunch(c->g_one, c->stream));
     }
-    while (left-- > 0) HIPCHK(c, hipGraphLaunch(c->g_one, c->stream));
     State12 st{};
     HIPCHK(c, hipMemcpyAsync(&st, c->b.st, sizeof st, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -11,8 +11,10 @@
 // row of D, and advance the step counter.
 #include "pic1d2v_internal.h"
 #include "pic_device.h"
+#include "seg16.h"
 #include "solve1d.h"
 #include "stencil1d.h"
+#include "wave_fft.h"
 
 #pragma clang fp contract(off)
 
@@ -172,14 +174,12 @@ k12_push(const Tile12* __restrict__ tiles, double* __restrict__ x, double* __res
     flush_limbs(acc, N, racc + (q < 0.0 ? 3 * N : 0));
 }
 
-// Diagnostics partials over chunks of 4096 particle indices, when t % bin == 0:
+// Diagnostics partials over chunk c of 4096 particle indices:
 // sum(vy^2 + vx^2 [+ M*(vy2^2 + vx2^2)]), sum(vx/P [+ M*vx2/P]), same for vy.
-__global__ void __launch_bounds__(256)
-k12_diag_chunks(const double* __restrict__ vx, const double* __restrict__ vy, int64_t P, int ns, double m0,
-                double m1, int bin, const State12* __restrict__ st, double* __restrict__ dpart) {
-    __shared__ double red[4 * kTreeLanes + 8];
-    if ((st->step + 1) % bin != 0) return;
-    const int64_t s = (int64_t)blockIdx.x * kTreeChunk;
+// red: LDS of 4*kTreeLanes + 8 doubles; every thread of the block calls.
+__device__ __forceinline__ void diag_chunk12(double* red, const double* vx, const double* vy, int64_t P, int ns,
+                                             double m0, double m1, int64_t chunk, double* dpart) {
+    const int64_t s = chunk * kTreeChunk;
     const int64_t n = P - s < kTreeChunk ? P - s : kTreeChunk;
     const double Pd = (double)P;
     double a = 0.0, b = 0.0, c = 0.0;
@@ -201,10 +201,19 @@ k12_diag_chunks(const double* __restrict__ vx, const double* __restrict__ vy, in
         }
     tree256x3<false>(red, a, b, c);
     if (threadIdx.x == 0) {
-        dpart[3 * blockIdx.x] = a;
-        dpart[3 * blockIdx.x + 1] = b;
-        dpart[3 * blockIdx.x + 2] = c;
+        dpart[0] = a;
+        dpart[1] = b;
+        dpart[2] = c;
     }
+}
+
+// the partials when t % bin == 0
+__global__ void __launch_bounds__(256)
+k12_diag_chunks(const double* __restrict__ vx, const double* __restrict__ vy, int64_t P, int ns, double m0,
+                double m1, int bin, const State12* __restrict__ st, double* __restrict__ dpart) {
+    __shared__ double red[4 * kTreeLanes + 8];
+    if ((st->step + 1) % bin != 0) return;
+    diag_chunk12(red, vx, vy, P, ns, m0, m1, blockIdx.x, dpart + 3 * blockIdx.x);
 }
 
 // Canonical tree over n values spread with stride 3 (in place).
@@ -222,28 +231,229 @@ __device__ double tree_stride3(double* red, double* vals, int64_t n) {
     return block_chunk_sum(red, n, [&](int64_t i) { return vals[3 * i]; });
 }
 
-// D[t/bin, 1:5] (src/NGP1D2V2S.jl:52-56) when t % bin == 0; then step += 1.
+// D[t/bin, 1:5] (src/NGP1D2V2S.jl:52-56) of step t, t % bin == 0, from the
+// chunk partials; every thread of the block calls.
+__device__ void diag_row12(double* red, double* dpart, int64_t nchunks, int64_t P, int N, double n0, int bin, int64_t t,
+                           double se, double* D, int64_t cap_bins) {
+    const double sk = tree_stride3(red, dpart, nchunks);
+    const double sx = tree_stride3(red, dpart + 1, nchunks);
+    const double sy = tree_stride3(red, dpart + 2, nchunks);
+    const int64_t bi = t / bin - 1;
+    if (threadIdx.x == 0 && bi < cap_bins) {
+        double* row = D + 5 * bi;
+        row[0] = row[0] + (se / (double)N) / 2.0;
+        row[1] = row[1] + ((sk * n0) / (double)P) / 2.0;
+        row[3] = row[3] + sx;
+        row[4] = row[4] + sy;
+        row[2] = row[2] + (row[0] + row[1]);
+        for (int c = 0; c < 3; ++c) row[c] = row[c] * (2.0 / n0);
+    }
+}
+
+// the row when t % bin == 0; then step += 1.
 __global__ void __launch_bounds__(256)
 k12_diag_final(double* __restrict__ dpart, int64_t nchunks, int64_t P, int N, double n0, int bin,
                State12* __restrict__ st, double* __restrict__ D, int64_t cap_bins) {
     __shared__ double red[kTreeLanes + 8];
     const int64_t t = st->step + 1;
-    if (t % bin == 0) {
-        const double sk = tree_stride3(red, dpart, nchunks);
-        const double sx = tree_stride3(red, dpart + 1, nchunks);
-        const double sy = tree_stride3(red, dpart + 2, nchunks);
-        const int64_t bi = t / bin - 1;
-        if (threadIdx.x == 0 && bi < cap_bins) {
-            double* row = D + 5 * bi;
-            row[0] = row[0] + (st->se / (double)N) / 2.0;
-            row[1] = row[1] + ((sk * n0) / (double)P) / 2.0;
-            row[3] = row[3] + sx;
-            row[4] = row[4] + sy;
-            row[2] = row[2] + (row[0] + row[1]);
-            for (int c = 0; c < 3; ++c) row[c] = row[c] * (2.0 / n0);
+    if (t % bin == 0) diag_row12(red, dpart, nchunks, P, N, n0, bin, t, st->se, D, cap_bins);
+    if (threadIdx.x == 0) st->step = t;
+}
+
+// ---------------------------------------------------------------------------
+// The FP64 step at the scripts' sizes (N <= kSmallN12, ns*P <= kSmallP12) in one
+// launch.  At some thousand particles the general chain's four launches are
+// latency: a push walks a particle's two stencils in one thread (15 us), the
+// solve is one block's LDS passes (10 us), and the two diagnostics launches
+// mostly end at their first test (2 x 4.5 us).  Here a particle takes a row of 16
+// lanes, and every block solves the field for itself in its first wave
+// (wave_fft.h) while the others evaluate their first particles' gather weights:
+// the launch boundary is the only meeting of the blocks.  Buffers that a launch
+// both reads and writes take turns: three charge accumulators (read, added to,
+// cleared) and two copies of the velocities, so that block 0, which has no
+// particles, can sum the velocities of the step before while this one's are
+// written.  The turn is the step number mod kSmallTurns12, known to the host.
+//
+// A chain of latencies bounds it: launch 3 us, loads 2, solve 4, fold and Boris
+// 0.6, the new stencil 1.6, adds 0.7.  2 x 2048 particles on 256 cells: 27.1 us a
+// step in the general chain, 13.4 here; 18.4 with the solve and the row in the
+// last block to arrive.  Every block adds its grid to the same words, and a CU
+// has few matches for its waves' erf chains: 32 particles a block 13.4 us, 16
+// 15.1, 48 13.6.
+// ---------------------------------------------------------------------------
+
+// E of the charge in sm (bit-reversed) into Eld, by a block's first wave, whose
+// lanes return their elements too.  sm: 3N doubles.
+template <int E>
+__device__ __forceinline__ void small_solve12(const double2* tw, int N, int log2N, double* sm,
+                                              double* Eld, double (&x)[E]) {
+    const int l = threadIdx.x & 63;
+    double* line = sm;
+    double* pr = sm + N;  // re, im
+    if (threadIdx.x >= 64) return;
+    const double* xi = reinterpret_cast<const double*>(tw) + kXiOffset;
+    double2 w6[6];
+    load_wave_twiddles(w6, tw, N);
+    double re[E], im[E], xt[E];
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int m = q * 64 + l;
+        re[q] = m < N ? line[m] : 0.0;
+        im[q] = 0.0;
+        xt[q] = m >= N ? 0.0 : m == 0 ? xi[1] : (m <= N / 2 ? xi[m] : -xi[N - m]);
+    }
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {  // one copy of the transform's code: it is fetched anew by each launch
+        wave_radix2<E>(re, im, w6, tw, N, pass != 0);
+        if (pass) break;
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int m = q * 64 + l;
+            if (m >= N) continue;
+            double a = im[q] * xt[q];
+            double b = -(re[q] * xt[q]);
+            if (m == 0) {
+                a = a * 0.0;
+                b = b * 0.0;
+            }
+            const int p = (int)brev((uint32_t)m, log2N);
+            pr[p] = a;
+            pr[N + p] = b;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int q = 0; q < E; ++q) {
+            const int i = q * 64 + l;
+            re[q] = i < N ? pr[i] : 0.0;
+            im[q] = i < N ? pr[N + i] : 0.0;
         }
     }
-    if (threadIdx.x == 0) st->step = t;
+    const double scale = 1.0 / (double)N;
+#pragma unroll
+    for (int q = 0; q < E; ++q) {
+        const int i = q * 64 + l;
+        x[q] = i < N ? re[q] * scale : 0.0;
+        if (i < N) Eld[i] = x[q];
+    }
+}
+
+// the D row of step t from the velocities after it, by a whole block
+__device__ void small_row12(const Buffers12& b, double* sm, int64_t t, double se, const double* vx, const double* vy) {
+    for (int64_t c = 0; c < b.nchunks; ++c) {
+        diag_chunk12(sm, vx, vy, b.P, b.ns, b.mass[0], b.mass[1], c, b.dpart + 3 * c);
+        __syncthreads();
+    }
+    diag_row12(sm, b.dpart, b.nchunks, b.P, b.N, b.n0, b.bin, t, se, b.D, b.cap_bins);
+    __syncthreads();
+}
+
+template <int R, int E>
+__global__ void __launch_bounds__(kSmallThreads12 + 64) k12_small_step(Buffers12 b, int turn) {
+    extern __shared__ double sm[];
+    static_assert(kSmallThreads12 + 64 >= kTreeLanes, "the row's trees");
+    constexpr int kSegs = kSmallThreads12 / kSegLanes;
+    const int N = b.N, e = threadIdx.x & (kSegLanes - 1);
+    double* Eld = sm;                                 // N
+    u64* acc = reinterpret_cast<u64*>(sm + N);        // the positive charge's limbs, then the negative's
+    double* line = sm + 7 * N;                        // 3N
+    const int64_t all = b.ns * b.P;
+    const double *vx0 = b.vx + (turn & 1) * all, *vy0 = b.vy + (turn & 1) * all;
+    double *vx1 = b.vx + (1 - (turn & 1)) * all, *vy1 = b.vy + (1 - (turn & 1)) * all;
+    u64* racc = (u64*)b.racc;
+    const u64* rd = racc + 6 * N * (turn % 3);
+    u64* add = racc + 6 * N * ((turn + 1) % 3);
+    u64* clr = racc + 6 * N * ((turn + 2) % 3);
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        const u128 pos = limbs_to_u128(rd[3 * i], rd[3 * i + 1], rd[3 * i + 2]),
+                   neg = limbs_to_u128(rd[3 * N + 3 * i], rd[3 * N + 3 * i + 1], rd[3 * N + 3 * i + 2]);
+        line[(int)brev((uint32_t)i, b.log2N)] = pos >= neg ? fxp_to(pos - neg, b.qbits) : -fxp_to(neg - pos, b.qbits);
+    }
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 6 * N; i += gridDim.x * blockDim.x) clr[i] = 0;
+    zero_lds(acc, 6 * N);
+    __syncthreads();
+    double x[E];
+    if (blockIdx.x == 0) {
+        const int64_t done = b.st->step;
+        const double se = b.st->se;
+        __syncthreads();  // read by all before lane 0 writes them
+        small_solve12<E>(b.tw, N, b.log2N, line, Eld, x);
+        if (threadIdx.x < 64) {
+            const int64_t bi = (done + b.bin) / b.bin - 1;  // of step done + 1
+            double y[2][E], r[2];
+#pragma unroll
+            for (int q = 0; q < E; ++q) {
+                const int i = q * 64 + threadIdx.x;
+                if (i < N && bi < b.cap_bins) b.Es[bi * N + i] = b.Es[bi * N + i] + x[q];
+                y[0][q] = fabs(x[q]);
+                y[1][q] = x[q] * x[q];
+            }
+            wave_canon<2, E>(r, y, [](int k, double a, double c) { return k < 1 ? nanmax(a, c) : a + c; });
+            if (threadIdx.x == 0) {
+                b.st->se = r[1];
+                if (!isfinite(r[0])) b.st->err |= 1;
+                b.st->step = done + 1;
+            }
+        }
+        if (done > 0 && done % b.bin == 0 && b.st->row != done) {
+            __syncthreads();
+            small_row12(b, sm, done, se, vx0, vy0);
+            if (threadIdx.x == 0) b.st->row = done;
+        }
+        return;
+    }
+    const double Nd = (double)N, iN = 1.0 / Nd;
+    const int64_t g0 = (int64_t)(blockIdx.x - 1) * kSegs + ((int)threadIdx.x >> 4) - 4;
+    const int64_t gs = (int64_t)(gridDim.x - 1) * kSegs;
+    double wt = 0.0, xj = 0.0;
+    int32_t first = 0;
+    if (threadIdx.x < 64) {
+        small_solve12<E>(b.tw, N, b.log2N, line, Eld, x);
+    } else if (g0 < all) {
+        xj = b.x[g0];
+        wt = seg_weight<R>(xj, Nd, iN, e, first, N - 1);
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) {
+        for (int64_t g = g0; g < all; g += gs) {
+            const int s = g >= b.P ? 1 : 0;
+            const double q = b.q[s];
+            double u = vx0[g], v = vy0[g];
+            if (g != g0) {
+                xj = b.x[g];
+                wt = seg_weight<R>(xj, Nd, iN, e, first, N - 1);
+            }
+            const double Ej = seg_fold<R>(Eld[(first + e) & (N - 1)] * wt);
+            boris12(u, v, Ej, b.B0, b.dt, b.q_m[s]);
+            const double xn = jl_mod1f(xj + u * b.dt);
+            if (e == 0) {
+                b.x[g] = xn;
+                vx1[g] = u;
+                vy1[g] = v;
+            }
+            int32_t to;
+            const double a = (q * seg_weight<R>(xn, Nd, iN, e, to, N - 1)) * b.w;
+            if (e <= 2 * R && fabs(a) > 0.0) {  // NaN adds nothing
+                const int32_t cell = (to + e) & (N - 1);
+                u64* r = acc + (q < 0.0 ? 3 * N : 0);
+                if (limbs_fit(q * b.w, b.qbits)) lds_add_contribution(r, N, cell, a, b.qbits);
+                else lds_add_fxp(r, N, cell, fxp_from(fabs(a), b.qbits));
+            }
+        }
+    }
+    __syncthreads();
+    flush_limbs(acc, N, add);
+    flush_limbs(acc + 3 * N, N, add + 3 * N);
+}
+
+// The row of the last step of a run, where its bin is full.
+__global__ void __launch_bounds__(256) k12_small_row(Buffers12 b, int turn) {
+    __shared__ double sm[4 * kTreeLanes + 8];
+    const int64_t done = b.st->step, all = b.ns * b.P;
+    small_row12(b, sm, done, b.st->se, b.vx + (turn & 1) * all, b.vy + (turn & 1) * all);
+    if (threadIdx.x == 0) b.st->row = done;
 }
 
 // rho from the exact signed charge (clearing it), for the deposit operator.
@@ -286,6 +496,22 @@ __global__ void k12_op_boris(double* __restrict__ vx, double* __restrict__ vy, c
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
+template <int E>
+static void small12(const Buffers12& b, int turn, hipStream_t s) {
+    const int64_t segs = kSmallThreads12 / kSegLanes, want = (b.ns * b.P + segs - 1) / segs;
+    const unsigned nb = 1 + (unsigned)(want < kSmallBlocks12 ? want : kSmallBlocks12);
+    const int words = 10 * b.N > 4 * kTreeLanes + 8 ? 10 * b.N : 4 * kTreeLanes + 8;  // the step's; the trees'
+    if (b.R == 6) k12_small_step<6, E><<<nb, kSmallThreads12 + 64, 8 * words, s>>>(b, turn);
+    else k12_small_step<7, E><<<nb, kSmallThreads12 + 64, 8 * words, s>>>(b, turn);
+}
+void launch12_small(const Buffers12& b, int turn, hipStream_t s) {
+    if (b.N <= 64) small12<1>(b, turn, s);
+    else if (b.N <= 128) small12<2>(b, turn, s);
+    else if (b.N <= 256) small12<4>(b, turn, s);
+    else small12<8>(b, turn, s);
+}
+void launch12_small_row(const Buffers12& b, int turn, hipStream_t s) { k12_small_row<<<1, 256, 0, s>>>(b, turn); }
+
 int push12_lds_bytes(int N) { return 32 * N; }  // E + three limb arrays
 
 void launch12_deposit(const Buffers12& b, hipStream_t s) {

@@ -21,6 +21,7 @@
 #include "fft_lines.h"
 #include "pic_device.h"
 #include "picem1d_internal.h"
+#include "seg16.h"
 #include "solve1d.h"
 #include "stencil1d.h"
 #include "wave_fft.h"
@@ -818,28 +819,6 @@ __global__ void __launch_bounds__(256) k_em_finish(EM1D s) {
 // ---------------------------------------------------------------------------
 constexpr int kEMSegs = kEMSmallThreads / 16;  // particles of a block at a time
 
-__device__ __forceinline__ u64 em_ld(const u64* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Whether this block is the last of the launch to arrive (all its threads call;
-// everything the others wrote before is visible then).  Clears the ticket.
-__device__ __forceinline__ bool em_last_block(uint32_t* ticket, int32_t* flag) {
-    wait_memory();  // every wave's adds have been made before thread 0 announces them
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const uint32_t n = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        *flag = n == gridDim.x - 1 ? 1 : 0;
-        if (*flag) {
-            __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        }
-    }
-    __syncthreads();
-    return *flag != 0;
-}
-
 // The exact grids of a block in LDS: grid g's lo and hi words (split50) at
 // 2 g N and (2 g + 1) N.  A contribution of at most M |w| goes there as u ff ws,
 // ws = w 2^q, where the split holds it (|t| < 2^101, see em_fits), else straight
@@ -879,7 +858,7 @@ __device__ __forceinline__ void em_flush50(const u64* lds, u64* dev, int N, int 
 }
 // the exact sum of a cell, read past this block's caches, and cleared
 __device__ __forceinline__ double em_take(u64* g, int N, int j, int q) {
-    const double v = em_sum(em_ld(g + j), em_ld(g + N + j), em_ld(g + 2 * N + j), q);
+    const double v = em_sum(ld_agent(g + j), ld_agent(g + N + j), ld_agent(g + 2 * N + j), q);
     g[j] = 0;
     g[N + j] = 0;
     g[2 * N + j] = 0;
@@ -1079,7 +1058,7 @@ __global__ void __launch_bounds__(kEMSmallThreads) k_ems_sweep(EM1D s, int sweep
     }
     __syncthreads();
     em_flush50(ldsu, s.racc, N, 3);
-    if (!em_last_block(s.ticket, &last)) return;
+    if (!last_block(s.ticket, &last)) return;
     const bool conv = em_wave_solve<E>(s, sweep, smd);
     if (threadIdx.x == 0) {
         s.ctl[kEMMaxSweeps] += 1;
@@ -1256,7 +1235,7 @@ __global__ void __launch_bounds__(kEMSmallThreads) k_ems_end(EM1D s) {
         __syncthreads();
         em_flush50(ldsu, s.racc + 9 * N, N, 7);
     }
-    if (!em_last_block(s.ticket, &last)) return;
+    if (!last_block(s.ticket, &last)) return;
     // the step's output slot (fields[:, t, 1:12]) and the next step's flags
     const int64_t slot = s.t[0] - s.t[1];
     const bool keep = slot >= 0 && slot < s.out_cap;

@@ -14,7 +14,16 @@ struct State12 {
     double se;     // sum(E.^2) of the latest field (canonical tree)
     int32_t err;   // bit 0: non-finite charge or field
     int32_t pad;
+    int64_t row;   // the one-launch step: the step whose D row was written last
 };
+
+// the FP64 step in one launch (kernels_1d2v.hip).  Beyond kSmallP12 particles the
+// general chain's threads are enough to hide their latency.
+constexpr int kSmallN12 = 512;
+constexpr int64_t kSmallP12 = 16384;  // particles of all species
+constexpr int kSmallThreads12 = 512;  // with particles, beside the solving wave
+constexpr int kSmallBlocks12 = 128;   // with particles
+constexpr int kSmallTurns12 = 6;      // the accumulators' three by the velocities' two
 
 // A run of at most `count` particles of one species from `start` in the
 // packed arrays (species s particle j at s*P + j), pushed by one workgroup.
@@ -29,8 +38,8 @@ struct Buffers12 {
     int64_t P;
     double q[2], q_m[2], mass[2];
     double w, n0, B0, dt;
-    double *x, *vx, *vy;           // ns*P each
-    unsigned long long* racc;      // 3 limbs per cell of the positive charge, then of the negative
+    double *x, *vx, *vy;           // ns*P each (small: twice the velocities)
+    unsigned long long* racc;      // 3 limbs per cell of the positive charge, then of the negative (small: three of them)
     double* E;                     // N
     double* Es;                    // cap_bins x N
     double* D;                     // cap_bins x 5
@@ -59,6 +68,9 @@ struct Buffers12 {
 
 int push12_lds_bytes(int N);
 void launch12_deposit(const Buffers12& b, hipStream_t s);  // the charge of the current positions
+// a whole step in one launch, turn = its number (from 0) mod kSmallTurns12; the D row of the steps before
+void launch12_small(const Buffers12& b, int turn, hipStream_t s);
+void launch12_small_row(const Buffers12& b, int turn, hipStream_t s);
 void launch12_solve(const Buffers12& b, hipStream_t s);    // E, binned E, sum(E.^2)
 void launch12_push(const Buffers12& b, hipStream_t s);     // gather, Boris, move, next charge
 void launch12_diag(const Buffers12& b, hipStream_t s);     // D row when t % bin == 0; step += 1

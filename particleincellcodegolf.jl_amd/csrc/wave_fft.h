@@ -1,4 +1,4 @@
-// wave_fft.h -- transforms of up to 256 points and the canonical norms inside one
+// wave_fft.h -- transforms of up to 512 points and the canonical norms inside one
 // wave, for the kernels whose small grids make them a latency chain: the lane
 // exchanges stay in registers (wave_ops.h), and so do a lane's twiddles.
 //
@@ -78,8 +78,8 @@ __device__ __forceinline__ void wave_radix2(double (&re)[E], double (&im)[E], co
 }
 
 // The canonical reduction tree (tree256 over lanes t < 256 that each fold the
-// elements t, t + 256, ... from +0.0) of K arrays of N <= 256 values in wave 0:
-// tree lane t = l + 64u folds slot u of lane l, the two halving steps combine
+// elements t, t + 256, ... from +0.0) of K arrays of N <= 512 values in one wave:
+// tree lane t = l + 64u folds slots u, u + 4 of lane l, the two halving steps combine
 // (u, u + 2) and then (0, 1) in lane l, and the last six steps are wave_tree's.
 // op(k, a, b): array k's sum or NaN-propagating maximum.  Every value is >= 0
 // (squares, magnitudes, flags), so folding +0.0 for a missing element leaves a
@@ -90,7 +90,11 @@ __device__ __forceinline__ void wave_canon(double (&r)[K], const double (&x)[K][
     for (int k = 0; k < K; ++k) {
         double P[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) P[u] = u < E ? op(k, 0.0, x[k][u < E ? u : 0]) : 0.0;
+        for (int u = 0; u < 4; ++u) {
+            P[u] = 0.0;
+#pragma unroll
+            for (int q = u; q < E; q += 4) P[u] = op(k, P[u], x[k][q]);
+        }
         r[k] = E > 2 ? op(k, op(k, P[0], P[2]), op(k, P[1], P[3])) : E > 1 ? op(k, P[0], P[1]) : P[0];
     }
     wave_tree<K>(r, op);
