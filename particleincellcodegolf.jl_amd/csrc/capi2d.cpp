@@ -35,7 +35,8 @@ struct pic2d_ctx {
     uint32_t *xq[2] = {}, *yq[2] = {}, *pid[2] = {};
     float *vx[2] = {}, *vy[2] = {}, *vz[2] = {};
     float *vxl[2] = {}, *vyl[2] = {}, *vzl[2] = {};
-    double *X64[2] = {}, *Y64[2] = {}, *VX64[2] = {}, *VY64[2] = {}, *VZ64[2] = {};
+    double *X64[2] = {}, *Y64[2] = {}, *VZ64[2] = {};
+    double2* V64[2] = {};
     // operator scratch (grown on demand)
     void* op[8] = {};
     size_t op_bytes[8] = {};
@@ -115,13 +116,11 @@ static void set_par(pic2d_ctx* c, int par) {
     c->par = par;
     b.X = c->X64[par];
     b.Y = c->Y64[par];
-    b.VX = c->VX64[par];
-    b.VY = c->VY64[par];
+    b.V = c->V64[par];
     b.VZ = c->VZ64[par];
     b.X_alt = c->X64[1 - par];
     b.Y_alt = c->Y64[1 - par];
-    b.VX_alt = c->VX64[1 - par];
-    b.VY_alt = c->VY64[1 - par];
+    b.V_alt = c->V64[1 - par];
     b.VZ_alt = c->VZ64[1 - par];
     b.Xq = c->xq[par];
     b.Yq = c->yq[par];
@@ -276,8 +275,7 @@ extern "C" int pic2d_create(pic2d_ctx** out, const pic2d_config* cfg) {
                 return fail(rc);
         } else {
             if ((rc = dalloc(c, &c->X64[k], P)) || (rc = dalloc(c, &c->Y64[k], P)) ||
-                (rc = dalloc(c, &c->VX64[k], P)) || (rc = dalloc(c, &c->VY64[k], P)) ||
-                (rc = dalloc(c, &c->VZ64[k], P)))
+                (rc = dalloc(c, &c->V64[k], P)) || (rc = dalloc(c, &c->VZ64[k], P)))
                 return fail(rc);
         }
     }
@@ -376,8 +374,11 @@ extern "C" int pic2d_upload(pic2d_ctx* c, const double* x, const double* y, cons
     } else {
         HIPCHK(c, hipMemcpy(b.X, x, 8 * P, hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(b.Y, y, 8 * P, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(b.VX, vx, 8 * P, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(b.VY, vy, 8 * P, hipMemcpyHostToDevice));
+        double* vxy = reinterpret_cast<double*>(b.V_alt);  // the two components, one after the other
+        HIPCHK(c, hipMemcpy(vxy, vx, 8 * P, hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(vxy + P, vy, 8 * P, hipMemcpyHostToDevice));
+        launch2d_pair(vxy, b.V, P, c->stream);
+        HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipMemcpy(b.VZ, vz, 8 * P, hipMemcpyHostToDevice));
         std::vector<uint32_t> q(P);
         for (int64_t p = 0; p < P; ++p) q[p] = (uint32_t)p;
@@ -428,7 +429,8 @@ extern "C" int pic2d_download(pic2d_ctx* c, double* x, double* y, double* vx, do
             list.push_back({kCopyPair32, vy, {b.VYf_alt, b.VYl_alt}, P, 1.0, nullptr});
             list.push_back({kCopyPair32, vz, {b.VZf_alt, b.VZl_alt}, P, 1.0, nullptr});
         } else {
-            const double* src[5] = {b.X_alt, b.Y_alt, b.VX_alt, b.VY_alt, b.VZ_alt};
+            const double* vxy = reinterpret_cast<double*>(b.V_alt);
+            const double* src[5] = {b.X_alt, b.Y_alt, vxy, vxy + P, b.VZ_alt};
             double* dst[5] = {x, y, vx, vy, vz};
             for (int k = 0; k < 5; ++k) list.push_back({kCopyF64, dst[k], {src[k], nullptr}, P, 1.0, nullptr});
         }

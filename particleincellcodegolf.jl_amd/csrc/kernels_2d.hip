@@ -460,9 +460,9 @@ k2d_tile_count64(Desc2D D, Tiles2D T, const double* __restrict__ X, const double
 // as k2d_tile_scatter; slot[i] gets the new slot of caller index i
 __global__ void __launch_bounds__(256)
 k2d_tile_scatter64(Desc2D D, Tiles2D T, const double* __restrict__ X, const double* __restrict__ Y,
-                   const double* __restrict__ VX, const double* __restrict__ VY, const double* __restrict__ VZ,
+                   const double2* __restrict__ V, const double* __restrict__ VZ,
                    const uint32_t* __restrict__ pid, double* __restrict__ Xo, double* __restrict__ Yo,
-                   double* __restrict__ VXo, double* __restrict__ VYo, double* __restrict__ VZo,
+                   double2* __restrict__ Vo, double* __restrict__ VZo,
                    uint32_t* __restrict__ pido, uint32_t* __restrict__ slot, int64_t per_block) {
     extern __shared__ int32_t hist[];
     for (int i = threadIdx.x; i < T.ntiles; i += blockDim.x) hist[i] = 0;
@@ -480,8 +480,7 @@ k2d_tile_scatter64(Desc2D D, Tiles2D T, const double* __restrict__ X, const doub
         const uint32_t id = pid[p];
         Xo[d] = x;
         Yo[d] = y;
-        VXo[d] = VX[p];
-        VYo[d] = VY[p];
+        Vo[d] = V[p];
         VZo[d] = VZ[p];
         pido[d] = id;
         slot[id] = (uint32_t)d;
@@ -489,8 +488,8 @@ k2d_tile_scatter64(Desc2D D, Tiles2D T, const double* __restrict__ X, const doub
 }
 
 __global__ void __launch_bounds__(kTileThreads)
-k2d_push64t(Desc2D D, Tiles2D T, double* __restrict__ X, double* __restrict__ Y, double* __restrict__ VX,
-            double* __restrict__ VY, double* __restrict__ VZ, const double* __restrict__ Ex,
+k2d_push64t(Desc2D D, Tiles2D T, double* __restrict__ X, double* __restrict__ Y, double2* __restrict__ V,
+            double* __restrict__ VZ, const double* __restrict__ Ex,
             const double* __restrict__ Ey, u64* __restrict__ racc, double dt, double B0) {
     constexpr int W = kTile2D + 2 * kHalo2D;
     __shared__ double exw[W * W], eyw[W * W];
@@ -515,7 +514,8 @@ k2d_push64t(Desc2D D, Tiles2D T, double* __restrict__ X, double* __restrict__ Y,
     const int64_t len = a1 - a0;
     const int64_t p0 = a0 + len * part / T.splits, p1 = a0 + len * (part + 1) / T.splits;
     for (int64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) {
-        double x = X[p], y = Y[p], vx = VX[p], vy = VY[p], vz = VZ[p];
+        const double2 v = V[p];
+        double x = X[p], y = Y[p], vx = v.x, vy = v.y, vz = VZ[p];
         {
             const Area64 ax = area64(x, D.NX, D.pairing), ay = area64(y, D.NY, D.pairing);
             const int32_t ci[2] = {ax.c0, ax.c1}, cj[2] = {ay.c0, ay.c1};
@@ -547,8 +547,7 @@ k2d_push64t(Desc2D D, Tiles2D T, double* __restrict__ X, double* __restrict__ Y,
         y = unimod1(y + vy * dt);
         X[p] = x;
         Y[p] = y;
-        VX[p] = vx;
-        VY[p] = vy;
+        V[p] = double2{vx, vy};
         VZ[p] = vz;
         // deposit64's contributions (wx*wy)*w, j outer, i inner
         const Area64 bx = area64(x, D.NX, D.pairing), by = area64(y, D.NY, D.pairing);
@@ -867,20 +866,23 @@ k2d_diag_grid(const double* __restrict__ Ex, const double* __restrict__ Ey, int6
     if (threadIdx.x == 0) gpart[blockIdx.x] = r;
 }
 
-// slot (may be NULL): where each caller index's particle is held, so that the
-// sums run in the caller's order
-template <typename T>
+// The particle sums in the caller's order.  held: V[slot[i]] holds particle i's
+// velocity; else VX and VY are.  The held reads go to random lines:
+// what bounds them is lines, one a particle for the pair (two arrays: 130 us at
+// 2^22 particles; 56 as pairs).
+template <bool HELD>
 __global__ void __launch_bounds__(256)
-k2d_diag_parts(const T* __restrict__ VX, const T* __restrict__ VY, int64_t P, double w, double* __restrict__ ppart,
-               const uint32_t* __restrict__ slot) {
+k2d_diag_parts(const double2* __restrict__ V, const uint32_t* __restrict__ slot, const double* __restrict__ VX,
+               const double* __restrict__ VY, int64_t P, double w, double* __restrict__ ppart) {
     __shared__ double red[3 * kTreeLanes + 8];
     const int64_t s = (int64_t)blockIdx.x * kTreeChunk;
     const int64_t n = P - s < kTreeChunk ? P - s : kTreeChunk;
     double a = 0.0, b = 0.0, c = 0.0;
     if (threadIdx.x < kTreeLanes)
+#pragma unroll 4
         for (int64_t i = threadIdx.x; i < n; i += kTreeLanes) {
-            const int64_t q = slot ? (int64_t)slot[s + i] : s + i;
-            const double vx = (double)VX[q], vy = (double)VY[q];
+            const double2 v = HELD ? V[slot[s + i]] : double2{VX[s + i], VY[s + i]};
+            const double vx = v.x, vy = v.y;
             a = a + (vx * vx + vy * vy) * w;
             b = b + vx;
             c = c + vy;
@@ -931,6 +933,24 @@ __global__ void __launch_bounds__(256) k2d_unpermute(Arrays2D<T, K> a, const uin
     }
 }
 
+// as k2d_unpermute; the velocity pairs as all vx, then all vy
+__global__ void __launch_bounds__(256) k2d_unpermute64(Buffers2D b, int64_t P) {
+    double* vxy = reinterpret_cast<double*>(b.V_alt);
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (int64_t)gridDim.x * blockDim.x) {
+        const uint32_t q = b.pid[p];
+        const double2 v = b.V[p];
+        b.X_alt[q] = b.X[p];
+        b.Y_alt[q] = b.Y[p];
+        vxy[q] = v.x;
+        vxy[P + q] = v.y;
+        b.VZ_alt[q] = b.VZ[p];
+    }
+}
+__global__ void __launch_bounds__(256) k2d_pair(const double* __restrict__ vxy, double2* __restrict__ V, int64_t P) {
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < P; p += (int64_t)gridDim.x * blockDim.x)
+        V[p] = double2{vxy[p], vxy[P + p]};
+}
+
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
@@ -947,7 +967,7 @@ void launch2d_push(const Buffers2D& b, hipStream_t s) {
             b.D, b.T, b.Xq, b.Yq, b.VXf, b.VYf, b.VZf, b.VXl, b.VYl, b.VZl, b.E32, b.racc, (float)(b.dt / 2.0), (float)t1,
             (float)tscale, (float)(b.dt * 4294967296.0));
     } else {
-        k2d_push64t<<<b.T.ntiles * b.T.splits, kTileThreads, 0, s>>>(b.D, b.T, b.X, b.Y, b.VX, b.VY, b.VZ, b.Ex, b.Ey,
+        k2d_push64t<<<b.T.ntiles * b.T.splits, kTileThreads, 0, s>>>(b.D, b.T, b.X, b.Y, b.V, b.VZ, b.Ex, b.Ey,
                                                                      b.racc, b.dt, b.B0);
     }
 }
@@ -965,9 +985,13 @@ void launch2d_tile_sort(const Buffers2D& b, hipStream_t s) {
     } else {
         k2d_tile_count64<<<nb, 256, lds, s>>>(b.D, b.T, b.X, b.Y);
         k2d_tile_scan<<<1, 1024, 0, s>>>(b.T);
-        k2d_tile_scatter64<<<nb, 256, lds, s>>>(b.D, b.T, b.X, b.Y, b.VX, b.VY, b.VZ, b.pid, b.X_alt, b.Y_alt,
-                                                b.VX_alt, b.VY_alt, b.VZ_alt, b.pid_alt, b.slot, per);
+        k2d_tile_scatter64<<<nb, 256, lds, s>>>(b.D, b.T, b.X, b.Y, b.V, b.VZ, b.pid, b.X_alt, b.Y_alt, b.V_alt,
+                                                b.VZ_alt, b.pid_alt, b.slot, per);
     }
+}
+
+void launch2d_pair(const double* vxy, double2* V, int64_t P, hipStream_t s) {
+    k2d_pair<<<push_blocks(P), 256, 0, s>>>(vxy, V, P);
 }
 
 void launch2d_unpermute(const Buffers2D& b, hipStream_t s) {
@@ -979,9 +1003,7 @@ void launch2d_unpermute(const Buffers2D& b, hipStream_t s) {
             {b.Xq_alt, b.Yq_alt, f(b.VXf_alt), f(b.VYf_alt), f(b.VZf_alt), f(b.VXl_alt), f(b.VYl_alt), f(b.VZl_alt)}};
         k2d_unpermute<uint32_t, 8><<<push_blocks(P), 256, 0, s>>>(a, b.pid, P);
     } else {
-        const Arrays2D<double, 5> a = {{b.X, b.Y, b.VX, b.VY, b.VZ},
-                                       {b.X_alt, b.Y_alt, b.VX_alt, b.VY_alt, b.VZ_alt}};
-        k2d_unpermute<double, 5><<<push_blocks(P), 256, 0, s>>>(a, b.pid, P);
+        k2d_unpermute64<<<push_blocks(P), 256, 0, s>>>(b, P);
     }
 }
 
@@ -1007,7 +1029,7 @@ void launch2d_diag_op(const double* Ex, const double* Ey, int64_t G, const doubl
                       double w, double* gpart, double* ppart, double* out, int64_t* drow, hipStream_t s) {
     const int64_t ng = (G + kTreeChunk - 1) / kTreeChunk, np = (P + kTreeChunk - 1) / kTreeChunk;
     k2d_diag_grid<<<(unsigned)ng, 256, 0, s>>>(Ex, Ey, G, gpart);
-    k2d_diag_parts<double><<<(unsigned)np, 256, 0, s>>>(vx, vy, P, w, ppart, nullptr);
+    k2d_diag_parts<false><<<(unsigned)np, 256, 0, s>>>(nullptr, nullptr, vx, vy, P, w, ppart);
     k2d_diag_final<<<1, 256, 0, s>>>(gpart, ng, ppart, np, G, P, out, drow, drow ? INT64_MAX : 1);
 }
 
@@ -1022,7 +1044,7 @@ void launch2d_diag(const Buffers2D& b, hipStream_t s) {
         k2d_diag_final32x<<<1, 256, 0, s>>>(b.gpart, ng, pp, np, G, P, b.D.w, b.diag, b.drow, b.diag_cap);
         return;
     }
-    k2d_diag_parts<double><<<(unsigned)np, 256, 0, s>>>(b.VX, b.VY, P, b.D.w, b.ppart, b.slot);
+    k2d_diag_parts<true><<<(unsigned)np, 256, 0, s>>>(b.V, b.slot, nullptr, nullptr, P, b.D.w, b.ppart);
     k2d_diag_final<<<1, 256, 0, s>>>(b.gpart, ng, b.ppart, np, G, P, b.diag, b.drow, b.diag_cap);
 }
 

@@ -48,7 +48,8 @@ struct Buffers2D {
     int blocks_push;
     double dt, B0;
     // particles (FP64 or mixed, by precision)
-    double *X, *Y, *VX, *VY, *VZ;
+    double *X, *Y, *VZ;
+    double2* V;              // FP64: (vx, vy), which the diagnostics read together in the caller's order
     uint32_t *Xq, *Yq;
     float *VXf, *VYf, *VZf;  // mixed: velocity hi words ...
     float *VXl, *VYl, *VZl;  // ... and lo words (v = hi + lo, |lo| <= ulp(hi)/2)
@@ -58,7 +59,8 @@ struct Buffers2D {
     uint32_t *Xq_alt, *Yq_alt, *pid_alt;
     float *VXf_alt, *VYf_alt, *VZf_alt;
     float *VXl_alt, *VYl_alt, *VZl_alt;
-    double *X_alt, *Y_alt, *VX_alt, *VY_alt, *VZ_alt;
+    double *X_alt, *Y_alt, *VZ_alt;
+    double2* V_alt;
     uint32_t* slot;          // FP64: the slot holding caller index i (diagnostics run in the caller's order)
     Tiles2D T;
     unsigned long long* racc;  // FP64: 3 limbs x NX*NY; mixed: NX*NY quanta
@@ -99,6 +101,8 @@ void launch2d_push(const Buffers2D& b, hipStream_t s);
 // mixed: regroup the held particles by tile into the _alt buffers
 void launch2d_tile_sort(const Buffers2D& b, hipStream_t s);
 // the particles in the caller's order, in the same format, into the alt buffers
+// (vx..., vy...) -> (vx, vy) pairs
+void launch2d_pair(const double* vxy, double2* V, int64_t P, hipStream_t s);
 void launch2d_unpermute(const Buffers2D& b, hipStream_t s);
 // src: 0 = FP64 limbs, 1 = mixed quanta, 2 = rho array, 3 = signed 38-bit limbs
 void launch2d_solve(const Buffers2D& b, int src, const double* rho_in, bool want_phi, hipStream_t s);
