@@ -815,21 +815,30 @@ __global__ void __launch_bounds__(256) k_lg_diag_field(LG23 L, int32_t buffer, i
     if (threadIdx.x == 0) L.fpart[blockIdx.x] = r;
 }
 
-// the field momentum's three sums over the cells (real parts of E and B)
+// the field momentum's three sums over the cells (real parts of E and B): few
+// blocks, so the loads of eight cells in flight (512 x 512: 24.0 us with a pass
+// for each sum, 11.9 in one)
 __global__ void __launch_bounds__(256) k_lg_diag_fmom(LG23 L, int64_t nch) {
-    __shared__ double red[kTreeLanes + 8];
+    __shared__ double red[3 * kTreeLanes + 8];
     const int64_t G = (int64_t)L.NX * L.NY;
     const int64_t s0 = (int64_t)blockIdx.x * kTreeChunk;
     const int64_t n = G - s0 < kTreeChunk ? G - s0 : kTreeChunk;
     const double2* F = L.F;
-    for (int c = 0; c < 3; ++c) {
-        const double r = block_chunk_sum(red, n, [&](int64_t i) {
-            const int64_t k = s0 + i;
-            const double Ex = F[kLGEx * G + k].x, Ey = F[kLGEy * G + k].x, Ez = F[kLGEz * G + k].x;
-            const double Bx = F[kLGBx * G + k].x, By = F[kLGBy * G + k].x, Bz = F[kLGBz * G + k].x;
-            return c == 0 ? Ey * Bz - Ez * By : (c == 1 ? Ez * Bx - Ex * Bz : Ex * By - Ey * Bx);
-        });
-        if (threadIdx.x == 0) L.mfpart[c * nch + blockIdx.x] = r;
+    double a = 0.0, b = 0.0, c = 0.0;
+#pragma unroll 8
+    for (int64_t i = threadIdx.x; i < n; i += kTreeLanes) {
+        const int64_t k = s0 + i;
+        const double Ex = F[kLGEx * G + k].x, Ey = F[kLGEy * G + k].x, Ez = F[kLGEz * G + k].x;
+        const double Bx = F[kLGBx * G + k].x, By = F[kLGBy * G + k].x, Bz = F[kLGBz * G + k].x;
+        a = a + (Ey * Bz - Ez * By);
+        b = b + (Ez * Bx - Ex * Bz);
+        c = c + (Ex * By - Ey * Bx);
+    }
+    tree256x3<false>(red, a, b, c);
+    if (threadIdx.x == 0) {
+        L.mfpart[blockIdx.x] = a;
+        L.mfpart[nch + blockIdx.x] = b;
+        L.mfpart[2 * nch + blockIdx.x] = c;
     }
 }
 
@@ -840,18 +849,29 @@ struct LGDiagFinal {
     double mass[kMaxSpecies23], weight[kMaxSpecies23];
 };
 
-__global__ void __launch_bounds__(256) k_lg_diag_final(LG23 L, Diag23 d, LGDiagFinal f) {
+// One block; the 4 + 7 ns trees one after the other took 28.5 us (two species of
+// 2^22 particles), side by side 12.8.
+__global__ void __launch_bounds__(1024) k_lg_diag_final(LG23 L, Diag23 d, LGDiagFinal f) {
     __shared__ double red[kTreeLanes + 8];
-    const double fe = tree_strided(red, L.fpart, 1, f.nfc) / (double)f.nf / 2.0;
+    // field energy and momenta; per species: kinetic, momenta, magnitudes
+    __shared__ double sum[4 + 7 * kMaxSpecies23];
+    tree_jobs(red, sum, 4 + 7 * f.ns, [&](int j) {
+        const int s = (j - 4) / 7, c = (j - 4) % 7 - 1;
+        if (j == 0) return TreeJob{L.fpart, 1, f.nfc};
+        if (j < 4) return TreeJob{L.mfpart + (j - 1) * f.nmc, 1, f.nmc};
+        return c < 0 ? TreeJob{d.kpart[s], 1, f.nk[s]} : TreeJob{d.mpart[s] + c, 6, f.nm[s]};
+    });
+    const double fe = sum[0] / (double)f.nf / 2.0;
     double fm[3];
-    for (int c = 0; c < 3; ++c) fm[c] = tree_strided(red, L.mfpart + c * f.nmc, 1, f.nmc) / (double)f.G;
+    for (int c = 0; c < 3; ++c) fm[c] = sum[1 + c] / (double)f.G;
     double ke = 0.0, pm[3] = {0.0, 0.0, 0.0}, pc[3] = {0.0, 0.0, 0.0};
     for (int s = 0; s < f.ns; ++s) {
-        const double kes = tree_strided(red, d.kpart[s], 1, f.nk[s]) * f.mass[s] / 2.0 * f.weight[s];
+        const double* sp = sum + 4 + 7 * s;
+        const double kes = sp[0] * f.mass[s] / 2.0 * f.weight[s];
         double ms[3], cs[3];
         for (int c = 0; c < 3; ++c) {
-            ms[c] = tree_strided(red, d.mpart[s] + c, 6, f.nm[s]) * (f.mass[s] * f.weight[s]);
-            cs[c] = tree_strided(red, d.mpart[s] + 3 + c, 6, f.nm[s]) * (f.mass[s] * f.weight[s]);
+            ms[c] = sp[1 + c] * (f.mass[s] * f.weight[s]);
+            cs[c] = sp[4 + c] * (f.mass[s] * f.weight[s]);
         }
         if (s == 0) {
             ke = kes;
@@ -902,7 +922,7 @@ void lg_launch_diag_row(const LG23& L, const Grid23& g, const Diag23& d, const S
         f.weight[s] = sp[s].weight;
         launch23_diag_species(sp[s], d.kpart[s], d.mpart[s], st);
     }
-    k_lg_diag_final<<<1, 256, 0, st>>>(L, d, f);
+    k_lg_diag_final<<<1, 1024, 0, st>>>(L, d, f);
 }
 
 // bins[a][t/ntskip][il, jl] += real(Z_a[il*g + ii, jl*g + jj]) * factor, jj

@@ -453,6 +453,50 @@ __device__ inline double tree_strided(double* red, double* vals, int stride, int
     return block_chunk_sum(red, n, [&](int64_t i) { return vals[stride * i]; });
 }
 
+// The canonical tree of n <= kTreeChunk values in one wave (lane 0 receives it):
+// lane l folds the tree lanes l, l + 64, l + 128 and l + 192.
+__device__ __forceinline__ double wave_tree_strided(const double* vals, int stride, int n) {
+    const int l = threadIdx.x & 63;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int i0 = 0; i0 < n; i0 += kTreeLanes)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = i0 + l + 64 * u;
+            const double x = vals[(int64_t)stride * (i < n ? i : n - 1)];
+            s[u] = s[u] + (i < n ? x : -0.0);
+        }
+    double r = (s[0] + s[2]) + (s[1] + s[3]);
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) r = r + __shfl_down(r, h, 64);
+    return r;
+}
+
+// The canonical trees of several arrays by one block, out[j] that of job(j):
+// a wave to each, so that their chains of a few microseconds run side by side;
+// arrays of more than a chunk of partials by the whole block.
+struct TreeJob {
+    double* vals;
+    int stride;
+    int64_t n;
+};
+template <typename F>
+__device__ __forceinline__ void tree_jobs(double* red, double* out, int jobs, F&& job) {
+    for (int j = threadIdx.x >> 6; j < jobs; j += blockDim.x >> 6) {
+        const TreeJob q = job(j);
+        if (q.n > kTreeChunk) continue;
+        const double r = wave_tree_strided(q.vals, q.stride, (int)q.n);
+        if ((threadIdx.x & 63) == 0) out[j] = r;
+    }
+    for (int j = 0; j < jobs; ++j) {
+        const TreeJob q = job(j);
+        if (q.n <= kTreeChunk) continue;
+        const double r = tree_strided(red, q.vals, q.stride, q.n);
+        if (threadIdx.x == 0) out[j] = r;
+    }
+    __syncthreads();
+}
+
 template <typename F>
 __device__ __forceinline__ double block_maxabs(double* red, int64_t n, F&& elem) {
     const int t = threadIdx.x;
