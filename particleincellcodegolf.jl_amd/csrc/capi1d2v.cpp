@@ -426,9 +426,11 @@ int pic1d2v_run(pic1d2v_ctx* c, int64_t nsteps, double* D) {
         // the graph's turns are those of a step number that kSmallTurns12 divides
         auto one = [&](int64_t step) { launch12_small(c->b, (int)(step % kSmallTurns12), c->stream); };
         const int64_t end = c->step + nsteps;
+        const int64_t aligned = (c->step + kSmallTurns12 - 1) / kSmallTurns12 * kSmallTurns12;
+        // captured before the first launch: a run that fails here has taken no step
+        if (end - aligned >= kSmallSteps12 && !c->g_many && (rc = capture(c, kSmallSteps12, &c->g_many))) return rc;
         int64_t at = c->step;
-        while (at < end && at % kSmallTurns12) one(at++);
-        if (end - at >= kSmallSteps12 && !c->g_many && (rc = capture(c, kSmallSteps12, &c->g_many))) return rc;
+        while (at < end && at < aligned) one(at++);
         for (; end - at >= kSmallSteps12; at += kSmallSteps12) HIPCHK(c, hipGraphLaunch(c->g_many, c->stream));
         while (at < end) one(at++);
         if (end % c->b.bin == 0) launch12_small_row(c->b, (int)(end % kSmallTurns12), c->stream);

@@ -277,9 +277,9 @@ k12_diag_final(double* __restrict__ dpart, int64_t nchunks, int64_t P, int N, do
 // A chain of latencies bounds it: launch 3 us, loads 2, solve 4, fold and Boris
 // 0.6, the new stencil 1.6, adds 0.7.  2 x 2048 particles on 256 cells: 27.1 us a
 // step in the general chain, 13.4 here; 18.4 with the solve and the row in the
-// last block to arrive.  Every block adds its grid to the same words, and a CU
-// has few matches for its waves' erf chains: 32 particles a block 13.4 us, 16
-// 15.1, 48 13.6.
+// last block to arrive.  Every block adds its grid to the same words, and more
+// waves in a block run their erf chains in turn: 32 particles a block 13.4 us,
+// 16 15.1, 48 13.6.
 // ---------------------------------------------------------------------------
 
 // E of the charge in sm (bit-reversed) into Eld, by a block's first wave, whose

@@ -521,19 +521,6 @@ __device__ __forceinline__ double block_maxabs(double* red, int64_t n, F&& elem)
     return tree256<true>(red, m);
 }
 
-// LinearAlgebra.norm (generic_norm2) with the canonical sum, n <= 4096.
-template <typename F>
-__device__ __forceinline__ double block_norm2(double* red, int64_t n, F&& elem) {
-    double m = block_maxabs(red, n, elem);
-    if (m == 0.0 || isinf(m)) return m;
-    if (isfinite((double)n * m * m) && m * m != 0.0) {
-        double s = block_chunk_sum(red, n, [&](int64_t i) { double x = elem(i); return x * x; });
-        return sqrt(s);
-    }
-    double s = block_chunk_sum(red, n, [&](int64_t i) { double q = fabs(elem(i)) / m; return q * q; });
-    return m * sqrt(s);
-}
-
 // Three canonical trees at once (sum or NaN-propagating max); red holds
 // >= 3*256 + 3 doubles.  Same operands per tree as tree256.
 template <bool MAX>
