@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "em_step_end.h"
 #include "fft_lines.h"
 #include "pic_device.h"
 #include "picem1d_internal.h"
@@ -1197,7 +1198,7 @@ __global__ void __launch_bounds__(kEMSmallThreads) k_ems_end(EM1D s) {
     __shared__ int32_t last;
     const int N = s.N, P = (int)s.P, e = threadIdx.x & 15;
     const double Nd = (double)N, iN = 1.0 / Nd;
-    EMGrid g[7];
+    EMGrid g[7] = {};
     if (MOMENTS) {
         for (int i = threadIdx.x; i < 14 * N; i += blockDim.x) ldsu[i] = 0;
         g[0] = em_grid(s, 1.0);
@@ -1236,30 +1237,16 @@ __global__ void __launch_bounds__(kEMSmallThreads) k_ems_end(EM1D s) {
         em_flush50(ldsu, s.racc + 9 * N, N, 7);
     }
     if (!last_block(s.ticket, &last)) return;
-    // the step's output slot (fields[:, t, 1:12]) and the next step's flags
-    const int64_t slot = s.t[0] - s.t[1];
-    const bool keep = slot >= 0 && slot < s.out_cap;
-    double* o = s.out + (keep ? slot : 0) * 12 * N;
-    for (int i = threadIdx.x; i < 12 * N; i += blockDim.x) {
-        const int f = i / N, j = i - f * N;
-        if (f < 5) {
-            const double* src = f == 0 ? s.Ex : f == 1 ? s.Ey : f == 2 ? s.Ez : f == 3 ? s.By : s.Bz;
-            if (keep) o[i] = src[j];
-        } else if (MOMENTS) {
-            int q = g[0].q;
-#pragma unroll
-            for (int k = 1; k < 7; ++k) q = f - 5 == k ? g[k].q : q;
-            const double v = em_take(s.racc + (9 + 3 * (f - 5)) * N, N, j, q);
-            if (keep) o[i] = v;
-        }
-    }
-    if (threadIdx.x == 0) {
-        if (keep) s.sweeps_out[slot] = s.ctl[kEMMaxSweeps];
-        s.t[0] += 1;
-        s.ctl[0] = 1;
-        for (int k = 1; k <= kEMMaxSweeps; ++k) s.ctl[k] = 0;
-        for (int k = 2; k < kEMMomentMax + 3; ++k) s.umax[k] = 0;
-    }
+    // values, not a reference to g, which would put g in scratch memory
+    const int q0 = g[0].q, q1 = g[1].q, q2 = g[2].q, q3 = g[3].q, q4 = g[4].q, q5 = g[5].q, q6 = g[6].q;
+    em_step_end(
+        s, threadIdx.x, blockDim.x, MOMENTS ? 12 : 5,
+        [=](int f, int j) {
+            if (f < 5) return (f == 0 ? s.Ex : f == 1 ? s.Ey : f == 2 ? s.Ez : f == 3 ? s.By : s.Bz)[j];
+            const int q = f == 5 ? q0 : f == 6 ? q1 : f == 7 ? q2 : f == 8 ? q3 : f == 9 ? q4 : f == 10 ? q5 : q6;
+            return em_take(s.racc + (9 + 3 * (f - 5)) * N, N, j, q);
+        },
+        [] { __syncthreads(); });
 }
 
 // ---------------------------------------------------------------------------
