@@ -19,7 +19,7 @@ LIB = os.path.join(LIB_DIR, "libpicgolf.so")
 ARCH = os.environ.get("PIC_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["kernels_1d.hip", "kernels_mixed.hip", "kernels_mixed_aux.hip", "kernels_small.hip", "noalloc.hip", "kernels_2d.hip", "kernels_1d2v.hip", "kernels_2d3v.hip", "kernels_2d3v_mixed.hip",
-           "kernels_2d3v_lg.hip", "kernels_em1d.hip", "hostcopy.hip", "capi.cpp", "capi2d.cpp", "capi1d2v.cpp", "capi2d3v.cpp",
+           "kernels_2d3v_lg.hip", "kernels_em1d.hip", "hostcopy_kernel.hip", "hostcopy.cpp", "capi.cpp", "capi2d.cpp", "capi1d2v.cpp", "capi2d3v.cpp",
            "capi_em1d.cpp"]
 
 

@@ -499,8 +499,7 @@ int pic_create_batch(pic_ctx** out, const pic_config* cfgs, int32_t n) {
         if ((rc = dalloc(c, &c->small_gacc, 9 * kSmallCopies * (size_t)c->hinst[0].N))) return fail(rc);
         if ((rc = dalloc(c, &c->small_bar, kSmallBarWords))) return fail(rc);
     }
-    hostcopy_retain(c->device);
-    c->staging = true;
+    c->staging = hostcopy_retain(c->device);
     *out = c;
     return PIC_OK;
 }
@@ -608,8 +607,7 @@ int pic_download(pic_ctx* c, int32_t inst, double* x, double* v, double* E) {
     const InstDesc& d = c->hinst[inst];
     const int par = (int)(c->steps_done & 1);
     const size_t P = (size_t)d.P;
-    // the stream's work is done before the copies, which run on streams of
-    // their own
+    // the stream's work is done before the copies, some of which run on another
     HIPCHK(c, hipStreamSynchronize(c->stream));
     CopyOut list[3] = {};
     if (c->precision == PIC_PREC_FP64) {
@@ -620,7 +618,7 @@ int pic_download(pic_ctx* c, int32_t inst, double* x, double* v, double* E) {
         list[1] = {kCopyPair32, v, {c->rb.Vh[par] + d.poff, c->rb.Vl[par] + d.poff}, P, d.inv_vstep, nullptr};
     }
     list[2] = {kCopyPickF64, E, {c->rb.E[0] + d.goff, c->rb.E[1] + d.goff}, (size_t)d.N, 1.0, &c->rb.st[inst].e_cur};
-    HIPCHK(c, copy_out(c->device, list, 3));
+    HIPCHK(c, copy_out(c->device, c->stream, list, 3));
     return PIC_OK;
 }
 

@@ -313,8 +313,7 @@ extern "C" int pic2d_create(pic2d_ctx** out, const pic2d_config* cfg) {
         hipMemset(b.Ex, 0, G * sizeof(double)) != hipSuccess || hipMemset(b.Ey, 0, G * sizeof(double)) != hipSuccess ||
         hipMemset(b.E32, 0, G * sizeof(float2)) != hipSuccess || hipDeviceSynchronize() != hipSuccess)
         return fail(PIC_EHIP);
-    hostcopy_retain(c->cfg.device);
-    c->staging = true;
+    c->staging = hostcopy_retain(c->cfg.device);
     *out = c;
     return PIC_OK;
 }
@@ -437,7 +436,7 @@ extern "C" int pic2d_download(pic2d_ctx* c, double* x, double* y, double* vx, do
     }
     list.push_back({kCopyF64, Ex, {b.Ex, nullptr}, G, 1.0, nullptr});
     list.push_back({kCopyF64, Ey, {b.Ey, nullptr}, G, 1.0, nullptr});
-    HIPCHK(c, copy_out(c->cfg.device, list.data(), (int)list.size()));
+    HIPCHK(c, copy_out(c->cfg.device, c->stream, list.data(), (int)list.size()));
     return PIC_OK;
 }
 

@@ -569,8 +569,7 @@ extern "C" int pic2d3v_create(pic2d3v_ctx** out, const pic2d3v_config* cfg) {
         L.ky = ky;
     }
     if ((rc = zero_state(c))) return fail(rc);
-    hostcopy_retain(c->cfg.device);
-    c->staging = true;
+    c->staging = hostcopy_retain(c->cfg.device);
     *out = c;
     return PIC_OK;
 }
@@ -645,7 +644,7 @@ extern "C" int pic2d3v_download(pic2d3v_ctx* c, int32_t s, double* xyv) {
     else launch23_pack(sp, (double*)st, c->stream);
     if ((rc = finish(c))) return rc;
     const CopyOut all = {kCopyF64, xyv, {st, nullptr}, 5 * (size_t)sp.P, 1.0, nullptr};
-    HIPCHK(c, copy_out(c->cfg.device, &all, 1));
+    HIPCHK(c, copy_out(c->cfg.device, c->stream, &all, 1));
     return PIC_OK;
 }
 
@@ -1105,7 +1104,7 @@ extern "C" int pic2d3v_fields(pic2d3v_ctx* c, double* Exs, double* Eys, double* 
     const CopyOut list[3] = {{kCopyF64, Exs, {c->d.Exs, nullptr}, n / 8, 1.0, nullptr},
                              {kCopyF64, Eys, {c->d.Eys, nullptr}, n / 8, 1.0, nullptr},
                              {kCopyF64, phis, {c->d.phis, nullptr}, n / 8, 1.0, nullptr}};
-    HIPCHK(c, copy_out(c->cfg.device, list, 3));
+    HIPCHK(c, copy_out(c->cfg.device, c->stream, list, 3));
     return PIC_OK;
 }
 
@@ -1244,7 +1243,7 @@ extern "C" int pic2d3v_lg_get(pic2d3v_ctx* c, int32_t which, double* z) {
     const size_t G = (size_t)c->cfg.NX * c->cfg.NY;
     if (int rc = finish(c)) return rc;
     const CopyOut all = {kCopyF64, z, {c->lg.F + which * G, nullptr}, 2 * G, 1.0, nullptr};
-    HIPCHK(c, copy_out(c->cfg.device, &all, 1));
+    HIPCHK(c, copy_out(c->cfg.device, c->stream, &all, 1));
     return PIC_OK;
 }
 

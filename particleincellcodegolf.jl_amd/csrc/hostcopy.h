@@ -1,5 +1,5 @@
 // hostcopy.h -- device-to-host copies of a context's state into the caller's
-// ordinary memory (hostcopy.cpp).
+// ordinary memory (hostcopy.cpp, hostcopy_kernel.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -25,13 +25,25 @@ struct CopyOut {
 };
 
 // Copies every array of the list (entries without dst are left out).  The
-// caller has synchronised with whatever wrote the sources.  Returns a HIP
-// error code (0: done); throws nothing.
-hipError_t copy_out(int device, const CopyOut* list, int count);
+// caller has set the device and synchronised with whatever wrote the sources;
+// stream is the caller's own.  Calls of several threads run side by side.
+// Returns a HIP error code (0: done); throws nothing.
+hipError_t copy_out(int device, hipStream_t stream, const CopyOut* list, int count);
 
 // The staging buffers exist while some context of the device does: a context
-// retains them once when it is made and releases them when it is destroyed.
-void hostcopy_retain(int device);
+// retains them once when it is made and, if that returned true, releases them
+// when it is destroyed.
+bool hostcopy_retain(int device);
 void hostcopy_release(int device);
+
+// A short list converted by one kernel; off[k]: the first element of array k
+// in out.
+constexpr int kSmallList = 8;
+struct SmallList {
+    CopyOut a[kSmallList];
+    size_t off[kSmallList + 1];
+    int n;
+};
+hipError_t launch_copy_small(const SmallList& l, double* out, hipStream_t stream);
 
 }  // namespace pic
