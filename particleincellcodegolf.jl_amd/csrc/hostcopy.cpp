@@ -28,6 +28,7 @@
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -109,12 +110,15 @@ struct Held {
     std::unique_ptr<Pool> pool;
     int users = 0;
 };
-constexpr int kMaxDevices = 16;
 std::mutex g_pools_m;
-Held g_pools[kMaxDevices];
+std::map<int, Held>& pools() {
+    static std::map<int, Held>* p = new std::map<int, Held>;  // lives as long as any context may
+    return *p;
+}
 Pool* pool_of(int device) {
     std::lock_guard<std::mutex> l(g_pools_m);
-    return g_pools[device].pool.get();
+    const auto it = pools().find(device);
+    return it == pools().end() ? nullptr : it->second.pool.get();
 }
 
 size_t element_bytes(CopyKind k) { return k == kCopyF64 || k == kCopyPickF64 ? 8 : 4; }
@@ -251,10 +255,9 @@ hipError_t copy_long(const Slab* slabs, int n, int device, hipStream_t stream, h
 }  // namespace
 
 bool hostcopy_retain(int device) {
-    if (device < 0 || device >= kMaxDevices) return false;
     try {
         std::lock_guard<std::mutex> l(g_pools_m);
-        Held& h = g_pools[device];
+        Held& h = pools()[device];
         if (!h.pool) h.pool.reset(new Pool);
         ++h.users;
         return true;
@@ -264,16 +267,15 @@ bool hostcopy_retain(int device) {
 }
 
 void hostcopy_release(int device) {
-    if (device < 0 || device >= kMaxDevices) return;
     std::unique_ptr<Pool> last;  // destroyed after the lock is given up
     std::lock_guard<std::mutex> l(g_pools_m);
-    Held& h = g_pools[device];
-    if (--h.users > 0) return;
-    last = std::move(h.pool);
+    const auto it = pools().find(device);
+    if (it == pools().end() || --it->second.users > 0) return;
+    last = std::move(it->second.pool);
+    pools().erase(it);
 }
 
 hipError_t copy_out(int device, hipStream_t stream, const CopyOut* list, int count) {
-    if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
     try {
         std::vector<CopyOut> items;
         size_t bytes = 0;

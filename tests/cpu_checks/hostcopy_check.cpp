@@ -231,6 +231,14 @@ int main() {
     expect(fake_pinned == 0 && fake_streams == 0 && fake_events == 0, "nothing is left");
     // no context holds the buffers
     formats(0, "not retained");
+    // every ordinal that a context may name
+    for (int device : {15, 16, 63}) {
+        expect(hostcopy_retain(device), "retained", device);
+        formats(device, "device");
+        expect(fake_pinned > 0, "staged", device);
+        hostcopy_release(device);
+    }
+    expect(fake_pinned == 0 && fake_streams == 0 && fake_events == 0, "nothing is left");
     std::printf("%d wrong\n", bad);
     return bad != 0;
 }
