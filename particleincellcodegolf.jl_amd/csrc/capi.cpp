@@ -16,6 +16,7 @@
 #include "../../include/pic.h"
 #include "hostcopy.h"
 #include "pic_internal.h"
+#include "tiling.h"
 #include "trace.h"
 
 using namespace pic;
@@ -252,32 +253,14 @@ const char* pic_last_error(const pic_ctx* ctx) {
     return ctx ? ctx->err.c_str() : g_create_err.c_str();
 }
 
-// Default tiling: every tile of every instance holds at most tileP particles.
-// FP64: as many tiles as fit at once (LDS-bound).  Mixed, one instance: one
-// 1024-thread block per CU below 8192 particles a block at two (a block's fixed
-// work -- its grid staged, cleared and flushed -- is then half the launch: 83.6
-// against 93.8 us a step at N = 1024, 3e5 particles; 158.8 against 163.1 at
-// N = 4096, 3e6), two beyond (353 against 365 us at 2^24).  Batches: 16 tiles of
-// 512 threads per CU, so that the ends of uneven instances and sweeps that only
-// some instances still need spread out, down to 1536 particles a tile (192
-// instances, 9.2e6 particles: 310 us a step with 2304-particle tiles, 387 with
-// 17984; 40 instances, 1.6e6 particles: 148 with 1664, 155 with 832).
-static void default_tiling(const pic_ctx* c, int64_t* tileP, int* block) {
+static Tiling default_tiling(const pic_ctx* c) {
     const int lds_push = c->scheme == PIC_SCHEME_SIMPSON
                              ? (c->precision == 0 ? simpson_push_lds_bytes(c->maxN) : simpson32_push_lds_bytes(c->maxN))
                              : push_lds_bytes(c->maxN, c->precision);
-    const int wg_per_cu = std::max(1, std::min(4, (160 * 1024) / std::max(lds_push, 1)));
-    auto per_tile = [&](int64_t tiles_per_cu) {
-        const int64_t target = (int64_t)c->numCU * tiles_per_cu;
-        return (c->Ptot + target - 1) / target;
-    };
-    if (c->ninst > 1) {
-        *tileP = std::max(per_tile(16), std::min<int64_t>(1536, per_tile(2)));
-        *block = 512;
-        return;
-    }
-    *tileP = c->precision == 0 ? per_tile(wg_per_cu) : per_tile(per_tile(2) < 8192 ? 1 : 2);
-    *block = (c->precision == 0 && wg_per_cu >= 2) ? 512 : 1024;
+    const int fit = std::max(1, std::min(4, (160 * 1024) / std::max(lds_push, 1)));
+    return choose_tiling(
+        c->ninst, [&](int i) { return c->cfg[i].N; }, [&](int i) { return c->cfg[i].P; }, c->precision == 0,
+        c->R == PIC_SHAPE_GAUSS6 || c->R == PIC_SHAPE_GAUSS7, fit, c->numCU);
 }
 
 // Lays the particles of every instance out in tiles of at most tileP (rounded
@@ -375,10 +358,8 @@ static int build_tables(pic_ctx* c) {
     if ((rc = dalloc(c, &b.insts, n))) return rc;
     if ((rc = dalloc(c, &b.st, n))) return rc;
     if ((rc = dalloc(c, &b.chunks, b.nchunks))) return rc;
-    int64_t tileP;
-    int block;
-    default_tiling(c, &tileP, &block);
-    if ((rc = layout_tiles(c, tileP, block))) return rc;
+    const Tiling tiling = default_tiling(c);
+    if ((rc = layout_tiles(c, tiling.tileP, tiling.block))) return rc;
     HIPCHK(c, hipMemcpy(b.chunks, c->hchunks.data(), sizeof(ChunkDesc) * b.nchunks, hipMemcpyHostToDevice));
     std::vector<InstState> st(n);
     for (auto& s : st) {
