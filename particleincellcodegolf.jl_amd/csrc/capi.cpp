@@ -260,7 +260,7 @@ static Tiling default_tiling(const pic_ctx* c) {
     const int fit = std::max(1, std::min(4, (160 * 1024) / std::max(lds_push, 1)));
     return choose_tiling(
         c->ninst, [&](int i) { return c->cfg[i].N; }, [&](int i) { return c->cfg[i].P; }, c->precision == 0,
-        c->R == PIC_SHAPE_GAUSS6 || c->R == PIC_SHAPE_GAUSS7, fit, c->numCU);
+        c->scheme == PIC_SCHEME_SIMPSON, c->R == PIC_SHAPE_GAUSS6 || c->R == PIC_SHAPE_GAUSS7, fit, c->numCU);
 }
 
 // Lays the particles of every instance out in tiles of at most tileP (rounded

@@ -13,10 +13,11 @@ struct Tiling {
 };
 
 // Members i = 0 .. n - 1 have cells(i) cells and particles(i) particles; fp64:
-// the precision; gauss: a Gaussian stencil; fit: workgroups whose LDS fits a CU
-// at once (1 .. 4).
+// the precision; simpson: the Simpson scheme; gauss: a Gaussian stencil; fit:
+// workgroups whose LDS fits a CU at once (1 .. 4).
 template <typename Cells, typename Particles>
-Tiling choose_tiling(int n, Cells&& cells, Particles&& particles, bool fp64, bool gauss, int fit, int numCU) {
+Tiling choose_tiling(int n, Cells&& cells, Particles&& particles, bool fp64, bool simpson, bool gauss, int fit,
+                     int numCU) {
     int64_t total = 0;
     double weighted = 0.0;  // sum of a particle's cells
     for (int i = 0; i < n; ++i) {
@@ -32,8 +33,10 @@ Tiling choose_tiling(int n, Cells&& cells, Particles&& particles, bool fp64, boo
     // (a block's fixed work -- its grid staged, cleared and flushed -- is then
     // half the launch: 83.6 against 93.8 us a step at N = 1024, 3e5 particles;
     // 158.8 against 163.1 at N = 4096, 3e6; two beyond: 353 against 365 us at
-    // 2^24).
-    const int per_cu = fp64 ? fit : (n == 1 && per_tile(2) < 8192 ? 1 : 2);
+    // 2^24).  The Simpson push has more work a particle: below 4096 (N = 64, 2e6
+    // particles: 238 against 239.5 us, 2.3e6: 260 against 253, 3.7e6: 339 against
+    // 327).
+    const int per_cu = fp64 ? fit : (n == 1 && per_tile(2) < (simpson ? 4096 : 8192) ? 1 : 2);
     const Tiling whole = {per_tile(per_cu), fp64 && fit >= 2 ? 512 : 1024};
     if (n == 1 || !gauss) return whole;
     // A batch whose members divide evenly runs all its tiles at once, and

@@ -21,8 +21,8 @@ def tiling(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", CSRC, os.path.join(ROOT, "tests", "cpu_checks", "tiling_check.cpp"),
                     "-o", str(exe)], check=True, timeout=120)
 
-    def run(members, fp64=False, gauss=True, fit=2):
-        args = [int(fp64), int(gauss), fit, CU] + [v for m in members for v in m]
+    def run(members, fp64=False, simpson=False, gauss=True, fit=2):
+        args = [int(fp64), int(simpson), int(gauss), fit, CU] + [v for m in members for v in m]
         return tuple(map(int, subprocess.run([str(exe)] + [str(a) for a in args], check=True, capture_output=True,
                                              text=True, timeout=30).stdout.split()))
     return run
@@ -71,6 +71,8 @@ def test_one_large_member_among_small_ones(tiling):
 def test_single_instances(tiling):
     assert tiling([(4096, 2 ** 24)]) == (2 ** 24 // 512, 1024)
     assert tiling([(4096, 3 * 10 ** 6)]) == (-(-3 * 10 ** 6 // 256), 1024)
+    assert tiling([(64, 3 * 10 ** 6)], simpson=True) == (-(-3 * 10 ** 6 // 512), 1024)
+    assert tiling([(64, 2 * 10 ** 6)], simpson=True) == (-(-2 * 10 ** 6 // 256), 1024)
     assert tiling([(4096, 3000001)], fp64=True, fit=1) == (-(-3000001 // 256), 1024)
     assert tiling([(1024, 10 ** 6)], fp64=True, fit=4) == (-(-10 ** 6 // 1024), 512)
     assert tiling([(64, 1)]) == (1, 1024)
