@@ -45,23 +45,31 @@ __device__ __forceinline__ int64_t em_irn(double c, int N) {
 
 // s(c) (:9-10): cells mod1(i, N) (0-based) and ff(i, c) for i = irn-6 .. irn+6.
 // Adjacent cells share an edge: ((i+1) - 0.5) equals (i + 0.5) exactly.  The
-// centre's cell wraps and c does not, so only a c within half a cell of its
-// wrapped cell has its edges in gauss_edges' intervals; any other is at least
-// N - 1/2 cells away, beyond 6 from every edge for N >= 16: all edges are
-// +-1/2 and the weights 0.
+// centre's cell wraps and c does not: where it wrapped by d cells, its edges are
+// those of the cell c lies in, d further on, and beyond these all edges are
+// +-1/2 and the weights 0 -- every weight for |d| >= 16, so for N >= 16.
+// (N = 8, 20000 particles in any order: 143 us a step; 227 with the edges of such
+// centres one by one, 219 with those of all centres.)
 __device__ __forceinline__ void em_stencil(double c, int N, double Nd, int32_t* cell, double* ff) {
     const int64_t i0 = em_irn(c, N);
     const double cN = c * Nd, r = rint(cN);
 #pragma unroll
     for (int k = 0; k < 13; ++k) cell[k] = (int32_t)((i0 - 6 + k - 1) & (int64_t)(N - 1));
-    if (edges_fit(cN) && (double)i0 == r) {
+    if (edges_fit(cN)) {
         double f[14];
         gauss_edges<6>(c, r, Nd, 1.0 / Nd, f);
 #pragma unroll
         for (int k = 0; k < 13; ++k) ff[k] = f[k + 1] - f[k];
-    } else if (edges_fit(cN) && N >= 16) {
+        const double d = (double)i0 - r;  // a multiple of N >= 8
+        if (d != 0.0) {
+            const bool up = d == 8.0, down = d == -8.0;
 #pragma unroll
-        for (int k = 0; k < 13; ++k) ff[k] = 0.0;
+            for (int k = 0; k < 8; ++k) {
+                const double lower = ff[k];
+                ff[k] = up && k < 5 ? ff[k + 8] : 0.0;
+                if (k < 5) ff[k + 8] = down ? lower : 0.0;
+            }
+        }
     } else {
         double lo = ol_erf((((double)(i0 - 6) - 0.5) / Nd - c) * Nd) / 2.0;
 #pragma unroll
