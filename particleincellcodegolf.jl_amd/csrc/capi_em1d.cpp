@@ -192,13 +192,13 @@ extern "C" int picem1d_create(picem1d_ctx** out, const picem1d_config* cfg) {
     // the short chain of kernels where none of them has work for the chip
     c->small = cfg->scheme == PICEM1D_FIXED_POINT && N <= kEMSmallN && P <= kEMSmallP &&
                cfg->max_sweeps <= kEMSmallSweeps;
-    if (c->small && !cfg->sort && (rc = dalloc(c, &s.tmp, 4 * (size_t)P))) return fail(rc);
-    if (cfg->sort) {
+    if ((c->small || cfg->sort) && (rc = dalloc(c, &s.tmp, 4 * (size_t)P))) return fail(rc);
+    if (cfg->sort && !c->small) {  // the small chain counts ranks in LDS
         const size_t B = (size_t)s.nb;
         if ((rc = dalloc(c, &s.count, B)) || (rc = dalloc(c, &s.cursor, B)) || (rc = dalloc(c, &s.start, B + 1)) ||
             (rc = dalloc(c, &s.bsum, 256)) || (rc = dalloc(c, &s.bucket, P)) || (rc = dalloc(c, &s.sidx, P)) ||
             (rc = dalloc(c, &s.sbucket, P)) || (rc = dalloc(c, &s.perm, P)) || (rc = dalloc(c, &s.vkey, P)) ||
-            (rc = dalloc(c, &s.skey, P)) || (rc = dalloc(c, &s.tmp, 4 * (size_t)P)))
+            (rc = dalloc(c, &s.skey, P)))
             return fail(rc);
     }
     const std::vector<double> twp = pass_twiddle_table();

@@ -1171,7 +1171,6 @@ __global__ void __launch_bounds__(kEMSmallThreads) k_ems_rank(EM1D s) {
         m[1] = fmax_num(m[1], fabs(v2));
         m[2] = fmax_num(m[2], fabs(v3));
         if (e < 4) s.tmp[(size_t)e * P + rank] = e == 0 ? jl_mod1f(s.x[p]) : e == 1 ? v1 : e == 2 ? v2 : v3;
-        if (SORT && e == 4) s.perm[rank] = (uint32_t)p;
     }
     em_block_max<3>(m, s.umax + kEMMomentMax, red);
 }
