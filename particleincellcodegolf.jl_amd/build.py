@@ -28,10 +28,13 @@ SOURCES = ["kernels_1d.hip", "kernels_mixed.hip", "kernels_mixed_aux.hip", "kern
 # over five alternating runs (instruction order only; the results are the
 # same bit for bit).  The mixed Simpson push ran about 5% slower under it,
 # so it lives in a unit of its own (kernels_mixed_aux.hip) without it.
-# The FP64 Gaussian units: hoisting the erf constants out of the particle loops spills
-# 103 scalar registers into vector lanes; without the hoisting the FP64
-# midpoint step (N = 4096, 3e6 particles) takes 1.00 in place of 1.03 ms, and
-# the 1D EM push needs 125 vector registers in place of 197.
+# The FP64 Gaussian units: hoisting the erf constants out of the particle loops
+# spills 103 scalar registers into vector lanes; without the hoisting the FP64
+# midpoint step (N = 4096, 3e6 particles) takes 1.00 in place of 1.03 ms, the
+# 1D EM push needs 125 vector registers in place of 197, 2048 steps of the 1D2V
+# script 27.7 in place of 28.6 ms, and the persistent midpoint run at N = 256,
+# 12288 particles (300 steps) 24.4 in place of 25.1 (at the script's size 71.3
+# both ways).
 EXTRA_FLAGS = {"kernels_1d.hip": ["-mllvm", "-disable-machine-licm"],
                "kernels_1d2v.hip": ["-mllvm", "-disable-machine-licm"],
                "kernels_em1d.hip": ["-mllvm", "-disable-machine-licm"],

@@ -22,7 +22,9 @@ constexpr int kLimbEM = 38;         // exact sums: three 38-bit two's-complement
 constexpr int kEMMaxSweeps = 8;     // ctl[s] = sweep s active; ctl[kEMMaxSweeps] = sweeps run this step
 
 // the small chain of the fixed point (see kernels_em1d.hip): at most this many
-// cells (a line in a wave), particles (their keys in LDS) and sweeps
+// cells (a line in a wave), particles (their keys in LDS) and sweeps.  At the
+// limits it is still the faster one: N = 256, 4096 particles, 131 us a step (136
+// allowed four sweeps, 117 unsorted) against the general chain's 243 (249, 156).
 constexpr int kEMSmallN = 256;
 constexpr int kEMSmallP = 4096;
 constexpr int kEMSmallSweeps = 4;
