@@ -24,6 +24,26 @@
 // deposit stencil each): 2370 vector instructions per wave in place of 6000,
 // 300 us a launch in place of 697, at 72% of the vector issue rate (four waves
 // per SIMD: the charge's LDS limbs fill the CU with one block).
+//
+// The forms and their constants restate FreeBSD msun e_exp.c and s_erf.c, whose
+// copyright notices are kept here as their licence asks:
+//
+// ====================================================
+// Copyright (C) 1993 by Sun Microsystems, Inc. All rights reserved.
+//
+// Developed at SunPro, a Sun Microsystems, Inc. business.
+// Permission to use, copy, modify, and distribute this
+// software is freely granted, provided that this notice
+// is preserved.
+// ====================================================
+//
+// ====================================================
+// Copyright (C) 2004 by Sun Microsystems, Inc. All rights reserved.
+//
+// Permission to use, copy, modify, and distribute this
+// software is freely granted, provided that this notice
+// is preserved.
+// ====================================================
 #pragma once
 #include "erfc_tail.h"
 #include "pic_device.h"
