@@ -209,8 +209,9 @@ PIC_HD double erf_tail_full(double x0) {
 // The polynomial's distance from msun's r/x in [M, M+1] is below tail_delta(M):
 // in [3, 4] both carry a few roundings of a value below 2.21e-5 (8 units in its
 // last place are 4.2e-20), beyond 4 the interpolation error of 1e-21 is the
-// larger part.  Over 2e9 random arguments per interval the two rounded
-// differently up to 1.0e-20, 8.5e-22 and 9.7e-22 from the middle of two doubles.
+// larger part.  Over 4e9 random arguments per interval the two rounded
+// differently up to 1.02e-20, 8.5e-22 and 9.8e-22 from the middle of two doubles
+// (tests/cpu_checks/gauss_edges_check.hip with an argument).
 PIC_HD constexpr double tail_delta(int M) { return M == 3 ? 4.2e-20 : 4.0e-21; }
 
 // erf(x) for x in [M, M+1], M = 3, 4, 5; the bits of unsure (from bit `at` on)

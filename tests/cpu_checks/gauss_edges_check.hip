@@ -2,9 +2,18 @@
 // on random arguments and around the branch points, whole stencils (R = 6, 7)
 // at random centres, cell edges and cell centres, and the limb split of a
 // contribution against fxp_from's definition on 128-bit integers.
+//
+// With an argument n: the measurement behind tail_delta.  Over n random
+// arguments in each of [3, 4], [4, 5] and [5, 6], the largest distance of
+// 1 - erfc from the middle of two doubles at which the polynomial's rounding
+// differs from the restatement's; fails where it exceeds tail_delta.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
 #include <random>
+#include <thread>
+#include <vector>
 
 #include "gauss_edges.h"
 
@@ -52,7 +61,51 @@ static void stencil(double c, int N) {
     }
 }
 
-int main() {
+template <int M>
+static void tail_sweep(long long count, unsigned seed, double* most, long long* differ) {
+    std::mt19937_64 rng(seed);
+    double far = 0.0;
+    long long d = 0;
+    for (long long i = 0; i < count; ++i) {
+        const double x = M + (double)(rng() >> 11) * 0x1p-53, u = x - (M + 0.5);
+        const double a = M == 3 ? erfc_tail3(u) : M == 4 ? erfc_tail4(u) : erfc_tail5(u);
+        const double y = 1.0 - a;
+        if (y == orc_erf(x)) continue;
+        ++d;
+        const double at = 0x1p-54 - std::fabs((1.0 - y) - a);
+        far = at > far ? at : far;
+    }
+    *most = far;
+    *differ = d;
+}
+static int tail_sweeps(long long count) {
+    const int T = (int)std::max(1u, std::thread::hardware_concurrency());
+    int wrong = 0;
+    for (int M = 3; M < 6; ++M) {
+        std::vector<double> most(T);
+        std::vector<long long> differ(T);
+        std::vector<std::thread> ts;
+        for (int t = 0; t < T; ++t) {
+            const long long n = count / T + (t < count % T);
+            auto f = M == 3 ? tail_sweep<3> : M == 4 ? tail_sweep<4> : tail_sweep<5>;
+            ts.emplace_back(f, n, 100u * M + t, &most[t], &differ[t]);
+        }
+        double far = 0.0;
+        long long d = 0;
+        for (int t = 0; t < T; ++t) {
+            ts[t].join();
+            far = std::max(far, most[t]);
+            d += differ[t];
+        }
+        std::printf("[%d, %d]: %lld arguments, %lld round differently, up to %.2e from the middle (tail_delta %.1e)\n",
+                    M, M + 1, count, d, far, tail_delta(M));
+        wrong += far > tail_delta(M);
+    }
+    return wrong;
+}
+
+int main(int argc, char** argv) {
+    if (argc > 1) return tail_sweeps(std::atoll(argv[1]));
     std::mt19937_64 rng(7);
     std::uniform_real_distribution<double> u(0.0, 1.0);
     for (int i = 0; i < 2000000; ++i)
