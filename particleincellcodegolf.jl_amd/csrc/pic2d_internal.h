@@ -98,11 +98,12 @@ inline size_t cols_lds_bytes(int NX, int NY) {
 
 // one time step: push + deposit, then the field solve
 void launch2d_push(const Buffers2D& b, hipStream_t s);
-// mixed: regroup the held particles by tile into the _alt buffers
+// regroup the held particles by tile into the _alt buffers
 void launch2d_tile_sort(const Buffers2D& b, hipStream_t s);
-// the particles in the caller's order, in the same format, into the alt buffers
 // (vx..., vy...) -> (vx, vy) pairs
 void launch2d_pair(const double* vxy, double2* V, int64_t P, hipStream_t s);
+// the particles into the alt buffers in the caller's order, in the same format
+// (the FP64 velocity pairs as all vx, then all vy)
 void launch2d_unpermute(const Buffers2D& b, hipStream_t s);
 // src: 0 = FP64 limbs, 1 = mixed quanta, 2 = rho array, 3 = signed 38-bit limbs
 void launch2d_solve(const Buffers2D& b, int src, const double* rho_in, bool want_phi, hipStream_t s);
