@@ -588,8 +588,6 @@ int pic_download(pic_ctx* c, int32_t inst, double* x, double* v, double* E) {
     const InstDesc& d = c->hinst[inst];
     const int par = (int)(c->steps_done & 1);
     const size_t P = (size_t)d.P;
-    // the stream's work is done before the copies, some of which run on another
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     CopyOut list[3] = {};
     if (c->precision == PIC_PREC_FP64) {
         list[0] = {kCopyF64, x, {c->rb.X[par] + d.poff, nullptr}, P, 1.0, nullptr};

@@ -411,7 +411,6 @@ extern "C" int pic2d_download(pic2d_ctx* c, double* x, double* y, double* vx, do
         return PIC_ESTATE;
     }
     HIPCHK(c, hipSetDevice(c->cfg.device));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     const size_t P = (size_t)c->cfg.P, G = (size_t)c->cfg.NX * c->cfg.NY;
     Buffers2D& b = c->b;
     std::vector<CopyOut> list;
@@ -420,7 +419,6 @@ extern "C" int pic2d_download(pic2d_ctx* c, double* x, double* y, double* vx, do
         // them in the caller's order
         launch2d_unpermute(b, c->stream);
         HIPCHK(c, hipGetLastError());
-        HIPCHK(c, hipStreamSynchronize(c->stream));
         if (c->cfg.precision == PIC_PREC_MIXED) {
             list.push_back({kCopyUnimod32, x, {b.Xq_alt, nullptr}, P, 1.0, nullptr});
             list.push_back({kCopyUnimod32, y, {b.Yq_alt, nullptr}, P, 1.0, nullptr});

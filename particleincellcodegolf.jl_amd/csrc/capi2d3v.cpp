@@ -642,7 +642,7 @@ extern "C" int pic2d3v_download(pic2d3v_ctx* c, int32_t s, double* xyv) {
     if ((rc = scratch(c, 0, sizeof(double) * 5 * (size_t)sp.P, &st))) return rc;
     if (c->mixed) launch23m_pack(c->g, sp, (double*)st, c->stream);
     else launch23_pack(sp, (double*)st, c->stream);
-    if ((rc = finish(c))) return rc;
+    HIPCHK(c, hipGetLastError());
     const CopyOut all = {kCopyF64, xyv, {st, nullptr}, 5 * (size_t)sp.P, 1.0, nullptr};
     HIPCHK(c, copy_out(c->cfg.device, c->stream, &all, 1));
     return PIC_OK;
@@ -1100,7 +1100,6 @@ extern "C" int pic2d3v_fields(pic2d3v_ctx* c, double* Exs, double* Eys, double* 
         if (phis) HIPCHK(c, hipMemcpy(phis, c->lg.bins + PIC2D3V_LG_BIN_PHI * blk, n, hipMemcpyDeviceToHost));
         return PIC_OK;
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     const CopyOut list[3] = {{kCopyF64, Exs, {c->d.Exs, nullptr}, n / 8, 1.0, nullptr},
                              {kCopyF64, Eys, {c->d.Eys, nullptr}, n / 8, 1.0, nullptr},
                              {kCopyF64, phis, {c->d.phis, nullptr}, n / 8, 1.0, nullptr}};
@@ -1241,7 +1240,6 @@ extern "C" int pic2d3v_lg_get(pic2d3v_ctx* c, int32_t which, double* z) {
     }
     HIPCHK(c, hipSetDevice(c->cfg.device));
     const size_t G = (size_t)c->cfg.NX * c->cfg.NY;
-    if (int rc = finish(c)) return rc;
     const CopyOut all = {kCopyF64, z, {c->lg.F + which * G, nullptr}, 2 * G, 1.0, nullptr};
     HIPCHK(c, copy_out(c->cfg.device, c->stream, &all, 1));
     return PIC_OK;

@@ -24,9 +24,9 @@ struct CopyOut {
     const int32_t* pick;
 };
 
-// Copies every array of the list (entries without dst are left out).  The
-// caller has set the device and synchronised with whatever wrote the sources;
-// stream is the caller's own.  Calls of several threads run side by side.
+// Copies every array of the list (entries without dst are left out) after the
+// work that stream, the caller's own, holds so far, which wrote the sources.
+// The caller has set the device.  Calls of several threads run side by side.
 // Returns a HIP error code (0: done); throws nothing.
 hipError_t copy_out(int device, hipStream_t stream, const CopyOut* list, int count);
 
