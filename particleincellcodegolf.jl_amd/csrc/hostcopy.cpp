@@ -17,10 +17,13 @@
 // caller's memory (32 KB: 11.5 us, and 15.9 through the kernel; 800 KB: 58 both
 // ways).
 //
-// A worker to every two slabs' worth of data, and the second stream for more
-// than two of them: making and freeing them costs some 0.1 ms each, which a
-// program with a context to a run pays every time (4e5 particles, 6.4 MB, from
-// create to destroy: 2.4 ms, with eight workers 3.2, in pageable memory 2.7).
+// A worker to every chunk; but a device's first two such copies make no more
+// slabs than one to every 4 MiB of theirs, and a second stream only for more than
+// two: making and freeing them costs some 0.1 ms each, which a program with a
+// context to a run, and a copy or two from it, would pay every time (4e5 FP64
+// particles, 6.4 MB, from create to destroy: 2.0 ms, with all at once 4.0, in
+// pageable memory 2.2).  A program that goes on reading gets them all (a grid of
+// 4 MiB in 0.30 ms; 0.65 by two, 0.69 in pageable memory).
 //
 // A copy takes the slabs that are free and never waits for another's: where
 // there is none (or no pinned memory to make one), it goes through pageable
@@ -45,6 +48,7 @@ constexpr int kWorkers = 8;                      // slabs one copy takes at most
 constexpr int kSlabs = 2 * kWorkers;             // slabs of a device, made when they are needed
 constexpr size_t kChunkBytes = size_t(1) << 20;  // of one pinned buffer
 constexpr size_t kSlabBytes = 2 * kChunkBytes;
+constexpr int kFirst = 2;                        // copies that make few slabs
 
 struct Slab {
     char* pin = nullptr;  // two buffers
@@ -61,10 +65,10 @@ void free_slab(Slab& s) {
 bool make_slab(Slab& s) {
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&s.pin), kSlabBytes, hipHostMallocDefault);
     if (e != hipSuccess) s.pin = nullptr;
-    // a waiting thread sleeps: the cores are the other workers' (spinning took
-    // as long)
+    // waited for by spinning: a sleeping thread wakes too late for a copy of a
+    // chunk or two (4 MiB by four: 0.30 ms, asleep 0.45 to 0.63)
     for (hipEvent_t& d : s.done)
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming | hipEventBlockingSync);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&d, hipEventDisableTiming);
     if (e == hipSuccess) return true;
     free_slab(s);
     (void)hipGetLastError();
@@ -75,28 +79,37 @@ bool make_slab(Slab& s) {
 struct Pool {
     std::mutex m;
     int made = 0;              // slabs that exist, free or taken
+    int copies = 0;            // by several workers so far
     Slab idle[kSlabs];         // the free ones
     int nidle = 0;
-    // every second worker's stream (the others take the caller's): with one
-    // stream, transfers and the waits for them queue behind each other (168 MB
-    // in 8.2 ms against 5.2 with eight); a further one costs a process 3 ms
-    hipStream_t second = nullptr;
+    // the workers' streams: with one, transfers and the waits for them queue
+    // behind each other (168 MB in 8.2 ms against 5.2 with eight); each costs a
+    // process 3 ms when it is first made.  A first copy's first one is the caller's.
+    hipStream_t own[2] = {nullptr, nullptr};
 
-    // up to `want` slabs; *other: the second stream, for more than two of them
-    int take(Slab* out, int want, hipStream_t* other = nullptr) {
+    void make_stream(hipStream_t& s) {
+        if (s || hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess) return;
+        s = nullptr;
+        (void)hipGetLastError();
+    }
+    // up to `want` slabs, of which a first copy makes those up to `few`; streams
+    // (the caller's, both, on entry): the ones to use in turn
+    int take(Slab* out, int want, int few = 1, hipStream_t* streams = nullptr) {
         std::lock_guard<std::mutex> l(m);
         int n = 0;
         while (n < want && nidle > 0) out[n++] = idle[--nidle];
-        for (; n < want && made < kSlabs; ++made)
+        const bool first = !streams || copies++ < kFirst;
+        const int make = first ? few : want;
+        for (; n < make && made < kSlabs; ++made)
             if (!make_slab(out[n++])) {
                 --n;
                 break;
             }
-        if (n > 2 && other && !second && hipStreamCreateWithFlags(&second, hipStreamNonBlocking) != hipSuccess) {
-            second = nullptr;
-            (void)hipGetLastError();
-        }
-        if (other) *other = second;
+        if (streams && n > (first ? 2 : 1)) make_stream(own[1]);
+        if (streams && n > 1 && !first) make_stream(own[0]);
+        if (streams && n > 1)
+            for (int k = 0; k < 2; ++k)
+                if (own[k]) streams[k] = own[k];
         return n;
     }
     void give(const Slab* s, int n) {
@@ -105,7 +118,8 @@ struct Pool {
     }
     ~Pool() {
         while (nidle > 0) free_slab(idle[--nidle]);
-        if (second) (void)hipStreamDestroy(second);
+        for (hipStream_t s : own)
+            if (s) (void)hipStreamDestroy(s);
     }
 };
 
@@ -241,19 +255,17 @@ hipError_t copy_small(const Slab& w, hipStream_t stream, const std::vector<CopyO
     return hipSuccess;
 }
 
-hipError_t copy_long(const Slab* slabs, int n, int device, hipStream_t stream, hipStream_t other,
-                     const std::vector<Chunk>& chunks) {
+hipError_t copy_long(const Slab* slabs, int n, int device, const hipStream_t* streams, const std::vector<Chunk>& chunks) {
     std::atomic<size_t> next(0);
     std::atomic<int> error(hipSuccess);
-    auto stream_of = [&](int k) { return (k & 1) && other ? other : stream; };
     std::vector<std::thread> threads;
     try {
         for (int k = 1; k < n; ++k)
-            threads.emplace_back([&, k] { work(slabs[k], stream_of(k), device, chunks, next, error); });
+            threads.emplace_back([&, k] { work(slabs[k], streams[k & 1], device, chunks, next, error); });
     } catch (...) {
         // fewer threads than asked for: the others take their chunks
     }
-    work(slabs[0], stream, device, chunks, next, error);
+    work(slabs[0], streams[0], device, chunks, next, error);
     for (std::thread& t : threads) t.join();
     return (hipError_t)error.load();
 }
@@ -315,15 +327,16 @@ hipError_t copy_out(int device, hipStream_t stream, const CopyOut* list, int cou
         }
         const unsigned hw = std::thread::hardware_concurrency();
         const size_t most = hw > 1 ? std::min<unsigned>(kWorkers, hw / 2) : 1;
-        const int want = (int)std::min(most, bytes / (2 * kSlabBytes) + 1);
+        const int want = (int)std::min(most, chunks.size());
+        const int few = (int)std::min(most, bytes / (2 * kSlabBytes) + 1);
         // the others' transfers do not wait for the caller's stream by themselves
         if (const hipError_t e = hipStreamSynchronize(stream)) return e;
-        hipStream_t other = nullptr;
-        const int n = p && bytes > kSlabBytes ? p->take(slabs, want, &other) : 0;
+        hipStream_t streams[2] = {stream, stream};
+        const int n = p && bytes > kSlabBytes ? p->take(slabs, want, few, streams) : 0;
         if (n == 0) return copy_plain(stream, chunks, items);
         hipError_t e = hipErrorOutOfMemory;
         try {
-            e = copy_long(slabs, n, device, stream, other, chunks);
+            e = copy_long(slabs, n, device, streams, chunks);
         } catch (...) {
         }
         p->give(slabs, n);

@@ -25,7 +25,7 @@ static std::map<void*, size_t> fake_pins;
 static size_t fake_pinned = 0, fake_most = 0;
 static int fake_streams = 0, fake_events = 0;
 static bool fail_pin = false, fail_stream = false, fail_event = false, fail_copy = false;
-static const void *gate_from = nullptr, *gate_to = nullptr;  // transfers from here wait
+static std::atomic<const void*> gate_from{nullptr}, gate_to{nullptr};  // transfers from here wait
 static int gate_waiting = 0;
 
 extern "C" {
@@ -182,7 +182,8 @@ static void beside(int device, size_t n) {
     expect(stuck.wait_for(std::chrono::seconds(0)) != std::future_status::ready, "the stuck copy is stuck");
     {
         std::lock_guard<std::mutex> l(fake_m);
-        gate_from = gate_to = nullptr;
+        gate_from = nullptr;
+        gate_to = nullptr;
     }
     fake_cv.notify_all();
     expect(stuck.get() == hipSuccess && other.get() == hipSuccess, "both copies end");
